@@ -187,7 +187,7 @@ int npbmz_tune(npbmz_ctx* ctx, int32_t budget_ms);
 #define NPBMZ_SCHED_LU_SWEEP 0   /* 0 hyperplane launches, 1 workgroup per zone,
                                     2 each zone's hyperplanes split by k rows over
                                     pipelined workgroups (tiles; FMA arithmetic,
-                                    where a tile's padded slots fit 512 threads;
+                                    where a workgroup's slots fit 448 threads;
                                     otherwise hyperplane launches).  Default
                                     with FMA arithmetic: 2 where a zone's padded
                                     hyperplane has more than 256 slots, else 1;
@@ -236,7 +236,9 @@ int npbmz_tune(npbmz_ctx* ctx, int32_t budget_ms);
 #define NPBMZ_SCHED_LU_TILES 7 /* LU pipelined sweep: tiles per zone, 1..8 (default:
                                   the padded slots over 256, rounded up, at most 8;
                                   4 where the tiles are not the default; fewer if a
-                                  zone has fewer padded k rows) */
+                                  zone has fewer padded k rows).  A tile runs as
+                                  several workgroups of at most 128 slots where the
+                                  device has CUs for them */
 #define NPBMZ_SCHED_LU_TILE_BATCH 8 /* LU pipelined sweep: hyperplanes a tile finishes
                                        between publishing its progress, 1..64
                                        (default 4) */

@@ -16,6 +16,7 @@
 #include <mutex>
 #include <numeric>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/npbmz.h"
@@ -224,7 +225,8 @@ constexpr int kMaxSolveGrid = 65536; // largest persistent solve grid accepted
 // workgroup per zone walking all hyperplanes of the sweep, or a zone's
 // hyperplanes split over pipelined workgroups (tiles).
 enum { kSweepPlane = 0, kSweepZone = 1, kSweepTiles = 2 };
-constexpr int kMaxTiles = 8;  // tiles per zone of the pipelined sweep
+constexpr int kMaxTiles = 8;    // tiles per zone of the pipelined sweep
+constexpr int kMaxGroups = 16;  // workgroups per zone its tiles may take
 
 // A task table on the device plus, per zone, the range of its tasks.
 struct Table {
@@ -268,7 +270,7 @@ struct npbmz_ctx {
   int lu_fwd = 3;                 // per-zone sweep: forward each hyperplane's rsd (1) and u (2)
                                   // through LDS; 3: the padded-halo sweep where it applies
   size_t max_lds = 65536;         // dynamic LDS a zone-sweep workgroup may take
-  int lu_tiles = 4;               // pipelined sweep: workgroups (tiles) per zone
+  int lu_tiles = 4;               // pipelined sweep: tiles per zone
   int lu_kb = 4;                  // pipelined sweep: hyperplanes per published count
   int lu_spin = 1 << 20;          // pipelined sweep: polls before a wait gives up
   int lu_handoff = -1;            // pipelined sweep: 0 agent-scope, 1 XCD-local, 2 XCD-local
@@ -420,6 +422,13 @@ LuK make_lu_constants(double dt, double omega, int nx0, int ny0, int nz0) {
     n.v_c1345 = v * k.c1345;
     n.v_ra = v * (k.r43 * k.c34 - k.c1345);
     n.v_rb = v * (k.c34 - k.c1345);
+    LuK::Push& q = k.push[d];
+    q.a = omega * a;
+    q.v = omega * v;
+    q.v_dd = q.v * dd[d];
+    q.v_c34 = q.v * k.c34;
+    q.v_r43c34 = q.v * k.r43 * k.c34;
+    q.v_m = q.v * (k.r43 - 1.0) * k.c34;
   }
   k.d0 = 1.0 + 2.0 * dt * (t1[0] * dd[0] + t1[1] * dd[1] + t1[2] * dd[2]);
   for (int i = 0; i < 3; ++i) {
@@ -432,6 +441,7 @@ LuK make_lu_constants(double dt, double omega, int nx0, int ny0, int nz0) {
     k.h[i] = 2.0 * dt * hs;
   }
   k.h5 = 2.0 * dt * k.c1345 * (t1[0] + t1[1] + t1[2]);
+  k.rd0 = 1.0 / k.d0;
   return k;
 }
 
@@ -849,22 +859,22 @@ int lu_fwd_level(const npbmz_ctx* c) {
   return lvl;
 }
 
-// Level 3, the padded-halo sweep with loads a hyperplane ahead: FMA
-// arithmetic, one padded (j, k) slot per thread, its LDS within the device's.
-size_t lu_halo_lds(const npbmz_ctx* c) {
-  return sizeof(double) * 2 * 10 * (size_t)(c->ny[0] - 1) * (c->nz[0] - 1);
-}
+// Level 3, the padded-halo sweep: FMA arithmetic, one padded (j, k) slot per
+// thread, its LDS (two hyperplanes of 10 doubles per thread) within the
+// device's.
+size_t lu_halo_lds(const npbmz_ctx* c) { return sizeof(double) * 2 * 10 * (size_t)c->lu_nt; }
 
 bool lu_halo_ok(const npbmz_ctx* c) {
   return c->lu_fwd == 3 && !(c->flags & NPBMZ_FLAG_STRICT_FP) &&
          (c->ny[0] - 1) * (c->nz[0] - 1) <= c->lu_nt && lu_halo_lds(c) <= c->max_lds;
 }
 
-// The pipelined tile sweep's shape: tiles per zone (none empty), slots per
-// tile, threads per workgroup (0 when a tile's slots exceed 512), hyperplane
-// steps and dynamic LDS.
+// The pipelined tile sweep's shape: a zone's slot rows are cut into W tiles
+// and each tile into `parts` workgroups of rpt rows, G workgroups in all
+// (none empty), each of nt slot threads (0 when no split fits) and a wave for
+// the hand-off; hyperplane steps and dynamic LDS.
 struct TileGeom {
-  int W, NS, nt, steps, SJ;
+  int W, parts, G, rpt, NS, nt, steps, SJ;
   size_t lds;
 };
 TileGeom tile_geom(const npbmz_ctx* c) {
@@ -872,13 +882,27 @@ TileGeom tile_geom(const npbmz_ctx* c) {
   const int NI = c->nx[0] - 2, NJ = c->ny[0] - 2, NK = c->nz[0] - 2;
   const int NR = NK + 1;
   g.SJ = NJ + 1;
-  int W = std::max(1, std::min(c->lu_tiles, NR));
-  const int rpt = (NR + W - 1) / W;
-  g.W = (NR + rpt - 1) / rpt;
-  g.NS = rpt * g.SJ;
-  g.nt = g.NS <= 128 ? 128 : g.NS <= 256 ? 256 : g.NS <= 512 ? 512 : 0;
-  g.steps = (NI + NJ + NK) & ~1;  // the halo hyperplane and ns interior ones, made even
-  g.lds = sizeof(double) * (2 * 10 * (size_t)g.NS + 1);  // the planes and one int
+  const int rows = (NR + c->lu_tiles - 1) / c->lu_tiles;  // of a tile
+  g.W = (NR + rows - 1) / rows;
+  // Workgroups of at most 128 slots, two waves: a step's loads and stores
+  // touch a cache line per slot, and more slots outrun their CU's L1 and its
+  // address processing.  Both sweeps, us, with workgroups of at most 128 and
+  // of 256 slots: class A (31x15 slots) 140 and 167, class B (51x16) 289 and
+  // 369, 64 zones of 29x13 171 and 189.  But no more of them than CUs, where
+  // a workgroup would only wait for a place (64 zones of 39x19: 4 of 195
+  // slots 540, 7 of 117 553), and none over 448 slots (with the hand-off
+  // wave, 8 waves, two a SIMD).
+  const int most = std::min(kMaxGroups, c->cus / ((c->nz_ + 7) & ~7));
+  int parts = (rows + std::max(1, 128 / g.SJ) - 1) / std::max(1, 128 / g.SJ);
+  parts = std::max(1, std::min(parts, most / g.W));
+  while (parts < rows && (rows + parts - 1) / parts * g.SJ > 448) ++parts;
+  g.rpt = (rows + parts - 1) / parts;
+  g.parts = (rows + g.rpt - 1) / g.rpt;
+  g.G = (NR + g.rpt - 1) / g.rpt;
+  g.NS = g.rpt * g.SJ;
+  g.nt = g.G > kMaxGroups ? 0 : g.NS <= 128 ? 128 : g.NS <= 256 ? 256 : g.NS <= 448 ? 448 : 0;
+  g.steps = NI + NJ + NK - 1;  // the halo hyperplane and the interior ones
+  g.lds = sizeof(double) * 2 * 15 * (size_t)g.nt;
   return g;
 }
 
@@ -917,15 +941,15 @@ bool xcd_round_robin() {
 }
 
 // Exchange rows and counters of the tile sweep, allocated once per context
-// for up to kMaxTiles tiles per zone, zeroed (each launch leaves them zero),
+// for up to kMaxGroups workgroups per zone, zeroed (each launch leaves them zero),
 // and the device's workgroup placement for the XCD-local hand-off.
 int ensure_tiles(npbmz_ctx* ctx) {
   auto& c = *ctx;
   if (c.txbuf) return NPBMZ_OK;
   c.tile_local_ok = xcd_round_robin();
   const TileGeom g = tile_geom(&c);
-  const size_t nx = (size_t)c.nz_ * kMaxTiles * g.steps * g.SJ * 10;
-  const size_t nc = (size_t)c.nz_ * kMaxTiles * 2 + c.nz_ + 1;
+  const size_t nx = (size_t)c.nz_ * kMaxGroups * g.steps * g.SJ * 5;
+  const size_t nc = (size_t)c.nz_ * kMaxGroups * 2 + c.nz_ + 1;
   double* xb = nullptr;
   int* cn = nullptr;
   hipError_t e = hipMalloc(&xb, nx * sizeof(double));
@@ -947,7 +971,7 @@ int ensure_tiles(npbmz_ctx* ctx) {
 int check_tiles(npbmz_ctx* ctx) {
   auto& c = *ctx;
   if (!c.tcnt) return NPBMZ_OK;
-  int* ef = c.tcnt + (size_t)c.nz_ * kMaxTiles + c.nz_;
+  int* ef = c.tcnt + (size_t)c.nz_ * kMaxGroups + c.nz_;
   int v = 0;
   CK(hipMemcpyAsync(&v, ef, sizeof v, hipMemcpyDeviceToHost, c.stream));
   CK(hipStreamSynchronize(c.stream));
@@ -984,46 +1008,40 @@ int k_lu_sweep_t(npbmz_ctx* ctx, int zone, bool* upd = nullptr) {
     if (!c.txbuf) return fail(ctx, NPBMZ_EHIP, "pipelined sweep buffers missing");
     const TileGeom g = tile_geom(&c);
     int* const cn = c.tcnt;
-    int* const dn = cn + (size_t)c.nz_ * kMaxTiles;
+    int* const dn = cn + (size_t)c.nz_ * kMaxGroups;
     int* const ef = dn + c.nz_;
-    // tile w of zone zl is block w * nzp + zl: the same residue mod 8 for all
-    // tiles of a zone
+    // workgroup w of zone zl is block w * nzp + zl: the same residue mod 8 for
+    // all of a zone
     const int nzp = (nzl + 7) & ~7;
     const int ho = tile_handoff(&c);
     int* const xc = ef + 1;
     auto go = [&](auto kern) {
-      hipLaunchKernelGGL(kern, dim3(nzp * g.W), dim3(g.nt), g.lds, c.stream, c.u, c.rhs, c.zd,
-                         z0, nzl, nzp, g.W, c.lu_kb, g.steps, c.txbuf, cn, dn, ef, c.lu_spin,
+      hipLaunchKernelGGL(kern, dim3(nzp * g.G), dim3(g.nt + 64), g.lds, c.stream, c.u, c.rhs, c.zd,
+                         z0, nzl, nzp, g.G, g.rpt, g.parts, c.lu_kb, g.steps, c.txbuf, cn, dn, ef, c.lu_spin,
                          xc, ho == 2 ? 1 : 0, c.lk);
     };
-    if (UPPER && upd) {
-      *upd = true;
-      if (ho != 0) {
-        switch (g.nt) {
-          case 128: go(fast::lu::sweep_tile_kernel<UPPER, 128, true, true>); break;
-          case 256: go(fast::lu::sweep_tile_kernel<UPPER, 256, true, true>); break;
-          default: go(fast::lu::sweep_tile_kernel<UPPER, 512, true, true>); break;
-        }
-      } else {
-        switch (g.nt) {
-          case 128: go(fast::lu::sweep_tile_kernel<UPPER, 128, false, true>); break;
-          case 256: go(fast::lu::sweep_tile_kernel<UPPER, 256, false, true>); break;
-          default: go(fast::lu::sweep_tile_kernel<UPPER, 512, false, true>); break;
-        }
-      }
-    } else if (ho != 0) {
-      switch (g.nt) {
-        case 128: go(fast::lu::sweep_tile_kernel<UPPER, 128, true>); break;
-        case 256: go(fast::lu::sweep_tile_kernel<UPPER, 256, true>); break;
-        default: go(fast::lu::sweep_tile_kernel<UPPER, 512, true>); break;
-      }
-    } else {
-      switch (g.nt) {
-        case 128: go(fast::lu::sweep_tile_kernel<UPPER, 128, false>); break;
-        case 256: go(fast::lu::sweep_tile_kernel<UPPER, 256, false>); break;
-        default: go(fast::lu::sweep_tile_kernel<UPPER, 512, false>); break;
-      }
-    }
+    // the hand-off form: XCD-local with 4 or 8 doubles of a row per lane, or
+    // agent-scope
+    auto by_form = [&](auto k4, auto k8, auto agent) {
+      if (ho == 0) go(agent);
+      else if (g.SJ * 5 <= 4 * 64) go(k4);
+      else go(k8);
+    };
+    auto by_size = [&](auto nt) {
+      constexpr int NT = decltype(nt)::value;
+      if (UPPER && upd)
+        by_form(fast::lu::sweep_tile_kernel<UPPER, NT, true, 4, true>,
+                fast::lu::sweep_tile_kernel<UPPER, NT, true, 8, true>,
+                fast::lu::sweep_tile_kernel<UPPER, NT, false, 8, true>);
+      else
+        by_form(fast::lu::sweep_tile_kernel<UPPER, NT, true, 4>,
+                fast::lu::sweep_tile_kernel<UPPER, NT, true, 8>,
+                fast::lu::sweep_tile_kernel<UPPER, NT, false, 8>);
+    };
+    if (g.nt == 128) by_size(std::integral_constant<int, 128>{});
+    else if (g.nt == 256) by_size(std::integral_constant<int, 256>{});
+    else by_size(std::integral_constant<int, 448>{});
+    if (UPPER && upd) *upd = true;
     CK(hipGetLastError());
     return NPBMZ_OK;
   }
@@ -1523,8 +1541,8 @@ void describe(npbmz_ctx* c) {
   char b[256];
   if (c->bench == NPBMZ_LU && c->lu_sweep == kSweepTiles && lu_tiles_ok(c)) {
     const TileGeom g = tile_geom(c);
-    snprintf(b, sizeof b, "zones=%d sweep=pipelined-tiles tiles=%d batch=%d nt=%d handoff=%s exch=%s fp=%s",
-             c->nz_, g.W, c->lu_kb, g.nt, tile_handoff(c) != 0 ? "xcd-local" : "agent",
+    snprintf(b, sizeof b, "zones=%d sweep=pipelined-tiles tiles=%d batch=%d nt=%d handoff=%s groups=%d exch=%s fp=%s",
+             c->nz_, g.W, c->lu_kb, g.nt * g.parts, tile_handoff(c) != 0 ? "xcd-local" : "agent", g.G,
              (c->flags & NPBMZ_FLAG_LU_NPB_EXCH) ? "npb" : "reference",
              strict(c) ? "strict" : "fma");
   } else if (c->bench == NPBMZ_LU)
@@ -1652,16 +1670,13 @@ int npbmz_create(const npbmz_problem* p, int32_t flags, npbmz_ctx** out) {
     if (interior > 32768) c.lu_sweep = kSweepPlane;
     else c.lu_nt = 512;
     // with FMA arithmetic, zones whose padded hyperplane exceeds 256 slots
-    // run as pipelined tiles of at most 256 slots each (below, npbmz_create:
-    // class A, 31x15 slots, 2 tiles: 0.300 ms per iteration against 0.327
-    // for the one-workgroup padded-halo sweep; class B, 51x16 slots, 4
-    // tiles: 0.686 against 1.095 with hyperplane launches; class W, 15x7
-    // slots, stays one workgroup per zone: 0.104 against 0.133 with 2 tiles)
+    // run as pipelined tiles of at most 256 slots each (below): both sweeps,
+    // us, one workgroup against tiles: class A (31x15 slots) 229 and 140;
+    // class B (51x16), whose hyperplane fits no workgroup, 1085 with
+    // hyperplane launches and 289.  Smaller ones gain little: 23x9 104 and 95,
+    // 19x11 83 and 86, class W (15x7) 47 and 60.
     // hyperplane forwarding: with FMA arithmetic the padded-halo sweep in
-    // the smallest workgroup that holds a zone's padded hyperplane (class W,
-    // 15x7 slots, 128 threads: 0.088 ms per iteration against 0.105 with 512
-    // threads from global memory; class S: 0.040 against 0.044; class A, 465
-    // slots, 512 threads: 0.351 against 0.533 from global memory); strict
+    // the smallest workgroup that holds a zone's padded hyperplane; strict
     // arithmetic has no padded-halo form: rsd and u through LDS from 128
     // (j, k) pairs up, else global memory
     const int hslots = (c.ny[0] - 1) * (c.nz[0] - 1);
@@ -1733,21 +1748,18 @@ int npbmz_create(const npbmz_problem* p, int32_t flags, npbmz_ctx** out) {
       grant(fast::lu::sweep_zone_kernel<false, 128, 2>); grant(fast::lu::sweep_zone_kernel<true, 128, 2>);
       grant(fast::lu::sweep_zone_kernel<false, 256, 2>); grant(fast::lu::sweep_zone_kernel<true, 256, 2>);
       grant(fast::lu::sweep_zone_kernel<false, 512, 2>); grant(fast::lu::sweep_zone_kernel<true, 512, 2>);
-      grant(fast::lu::sweep_zone_halo_kernel<false, 128>); grant(fast::lu::sweep_zone_halo_kernel<true, 128>);
-      grant(fast::lu::sweep_zone_halo_kernel<false, 256>); grant(fast::lu::sweep_zone_halo_kernel<true, 256>);
       grant(fast::lu::sweep_zone_halo_kernel<false, 512>); grant(fast::lu::sweep_zone_halo_kernel<true, 512>);
-      grant(fast::lu::sweep_tile_kernel<false, 128, false>); grant(fast::lu::sweep_tile_kernel<true, 128, false>);
-      grant(fast::lu::sweep_tile_kernel<false, 256, false>); grant(fast::lu::sweep_tile_kernel<true, 256, false>);
-      grant(fast::lu::sweep_tile_kernel<false, 512, false>); grant(fast::lu::sweep_tile_kernel<true, 512, false>);
-      grant(fast::lu::sweep_tile_kernel<false, 128, true>); grant(fast::lu::sweep_tile_kernel<true, 128, true>);
-      grant(fast::lu::sweep_tile_kernel<false, 256, true>); grant(fast::lu::sweep_tile_kernel<true, 256, true>);
-      grant(fast::lu::sweep_tile_kernel<false, 512, true>); grant(fast::lu::sweep_tile_kernel<true, 512, true>);
-      grant(fast::lu::sweep_zone_halo_kernel<true, 128, true>);
-      grant(fast::lu::sweep_zone_halo_kernel<true, 256, true>);
       grant(fast::lu::sweep_zone_halo_kernel<true, 512, true>);
-      grant(fast::lu::sweep_tile_kernel<true, 128, false, true>); grant(fast::lu::sweep_tile_kernel<true, 128, true, true>);
-      grant(fast::lu::sweep_tile_kernel<true, 256, false, true>); grant(fast::lu::sweep_tile_kernel<true, 256, true, true>);
-      grant(fast::lu::sweep_tile_kernel<true, 512, false, true>); grant(fast::lu::sweep_tile_kernel<true, 512, true, true>);
+      // (the padded sweeps' smaller workgroups take under 64 KiB)
+      grant(fast::lu::sweep_tile_kernel<false, 448, true, 4>);
+      grant(fast::lu::sweep_tile_kernel<false, 448, true, 8>);
+      grant(fast::lu::sweep_tile_kernel<false, 448, false, 8>);
+      grant(fast::lu::sweep_tile_kernel<true, 448, true, 4>);
+      grant(fast::lu::sweep_tile_kernel<true, 448, true, 8>);
+      grant(fast::lu::sweep_tile_kernel<true, 448, false, 8>);
+      grant(fast::lu::sweep_tile_kernel<true, 448, true, 4, true>);
+      grant(fast::lu::sweep_tile_kernel<true, 448, true, 8, true>);
+      grant(fast::lu::sweep_tile_kernel<true, 448, false, 8, true>);
       (void)hipGetLastError();
       if (ok) c.max_lds = (size_t)v;
     }
@@ -2182,7 +2194,7 @@ int npbmz_tune(npbmz_ctx* ctx, int32_t budget_ms) {
   if (c.bench == NPBMZ_LU) {
     knobs = {{NPBMZ_SCHED_LU_SWEEP, {1, 0, 2}}, {NPBMZ_SCHED_LU_THREADS, {128, 256, 512}},
              {NPBMZ_SCHED_LU_FORWARD, {3, 2, 1, 0}}, {NPBMZ_SCHED_LU_TILES, {2, 4, 8}},
-             {NPBMZ_SCHED_LU_TILE_BATCH, {2, 4, 8}}};
+             {NPBMZ_SCHED_LU_TILE_BATCH, {1, 2, 4}}};
   } else {
     knobs.push_back({-1, {1, 0}});
     if (c.bench == NPBMZ_BT) knobs.push_back({NPBMZ_SCHED_SOLVE_PAIR, {0, 2, 3, 7}});

@@ -66,6 +66,13 @@ struct LuK {
   // c1345) on direction i's t1 + (c34 - c1345) on the others); h5 = 2dt c1345
   // (tx1 + ty1 + tz1)
   double d0, g[3], h[3], h5;
+  // the products B(u) x of the padded sweeps (FMA arithmetic only), omega
+  // folded in: per direction a = omega*dt*t2, v = omega*dt*t1, v_dd = v*dd,
+  // v_c34 = v*c34, v_r43c34 = v*r43*c34, v_m = v*(r43-1)*c34; and 1/d0
+  struct Push {
+    double a, v, v_dd, v_c34, v_r43c34, v_m;
+  } push[3];
+  double rd0;
 };
 
 }  // namespace npbmz
