@@ -204,10 +204,13 @@ int npbmz_tune(npbmz_ctx* ctx, int32_t budget_ms);
                                     with a builder and an eliminator wave (default 2) */
 #define NPBMZ_SCHED_SOLVE_TWIST 4 /* BT and SP, FMA arithmetic only (ignored with
                                      NPBMZ_FLAG_STRICT_FP): bit d set: direction d
-                                     eliminates each line from both ends with two
-                                     waves meeting in the middle (BT: overrides
-                                     PAIR, default 7; SP: for directions whose
-                                     lines all have >= 6 points, default on where
+                                     eliminates each line from both ends, meeting
+                                     in the middle (BT: two waves per 64 lines,
+                                     overrides PAIR, default 7; SP: for directions
+                                     whose lines all have >= 6 points, six lines a
+                                     wave staged in LDS, default on where six of the
+                                     direction's lines fit it, up to 310 points;
+                                     longer lines two waves per 64, default on where
                                      the direction has fewer line tasks of 64
                                      lines than the device has CUs); the
                                      adjoint's transposed solves follow the

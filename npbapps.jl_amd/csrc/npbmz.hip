@@ -144,6 +144,7 @@ __device__ __forceinline__ double recip(double x) {
 #include "bt_rows.inc"
 #include "bt_adjoint.inc"
 #include "sp_kernels.inc"
+#include "sp_lines.inc"
 #include "sp_adjoint.inc"
 #include "lu_kernels.inc"
 #include "lu_adjoint.inc"
@@ -282,7 +283,10 @@ struct npbmz_ctx {
                                   // then per zone the tiles done, then the error flag,
                                   // then each tile's XCD plus one (XCD-local hand-off)
   Table t_int, t_all, t_line[3], t_face, t_face2;
-  Table t_row[3];  // BT: tasks of fast::bt::kRowLines lines for solve_rows_kernel
+  Table t_row[3];  // BT: tasks of fast::bt::kRowLines lines for solve_rows_kernel; SP: of
+                   // the staged solve's lines
+  bool sp_staged[3] = {false, false, false};  // SP, FMA only: the direction's lines fit
+                                              // solve_staged_kernel
   HaloSrc* hsrc = nullptr;  // BT/SP: where each zone side's halo cells come from
   bool hsrc_ok = false;     // hsrc describes the face table exactly
   int rhs_exch = 1;         // BT/SP batched steps: 1 exchange inside compute_rhs's launch
@@ -560,6 +564,10 @@ int build_tables(npbmz_ctx* ctx) {
       c.halfmax[d] = (mr + 1) / 2;
       const size_t spill_rows = (size_t)std::max(0, c.halfmax[d] - kRowR);
       slot = std::max(slot, (size_t)c.t_row[d].n * spill_rows * 2 * 6 * 64);
+    } else if (c.sp_staged[d]) {
+      if ((rc = build_table(ctx, c.t_row[d], ord, fast::sp::kStageLines,
+                            [&](int z) { return lines_of(ctx, z, d); })))
+        return rc;
     }
   }
   if (slot > c.cscr_slot) {
@@ -665,6 +673,11 @@ int build_tables(npbmz_ctx* ctx) {
   return NPBMZ_OK;
 }
 
+// LDS of SP's staged solve for lines of at most nl points.
+size_t staged_lds(int nl) {
+  return sizeof(double) * (size_t)fast::sp::kStageLines * fast::sp::staged_stride(nl);
+}
+
 bool strict(const npbmz_ctx* c) { return (c->flags & NPBMZ_FLAG_STRICT_FP) != 0; }
 
 // ------------------------------------------------------------ launches
@@ -740,6 +753,54 @@ bool rows_long(const npbmz_ctx& c, int d) {
   return c.t_row[d].n > 4 * c.cus && c.halfmax[d] > kRowRLong;
 }
 
+// Where SP runs the staged solve: lines of 6 points and more, six of which
+// fit a workgroup's LDS (up to 310 points in 160 KB).
+void choose_staged(npbmz_ctx& c) {
+  int dev = 0, lds = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess)
+    return;
+  bool ok = true;
+  auto grant = [&](auto kern) {
+    ok = ok && hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
+                                   hipFuncAttributeMaxDynamicSharedMemorySize, lds) == hipSuccess;
+  };
+  if (lds > 65536) {
+    grant(fast::sp::solve_staged_kernel<0, false>);
+    grant(fast::sp::solve_staged_kernel<1, false>);
+    grant(fast::sp::solve_staged_kernel<2, false>);
+    grant(fast::sp::solve_staged_kernel<2, true>);
+    grant(fast::sp::adj_solve_staged_kernel<0>);
+    grant(fast::sp::adj_solve_staged_kernel<1>);
+    grant(fast::sp::adj_solve_staged_kernel<2>);
+    (void)hipGetLastError();
+    if (!ok) lds = 65536;
+  }
+  for (int d = 0; d < 3; ++d) {
+    int nl = 0;
+    for (int z = 0; z < c.nz_; ++z)
+      nl = std::max(nl, d == 0 ? c.nx[z] : d == 1 ? c.ny[z] : c.nz[z]);
+    c.sp_staged[d] = c.sp_twist_ok[d] && staged_lds(nl) <= (size_t)lds;
+  }
+}
+
+// SP's staged solve of direction DIR over a task table's range, with LDS for
+// the direction's longest lines.
+template <int DIR, bool FUSE>
+int k_solve_staged(npbmz_ctx* ctx, int zone, double* xraw) {
+  auto& c = *ctx;
+  const Table& t = c.t_row[DIR];
+  const int first = zone < 0 ? 0 : t.zfirst[zone], n = zone < 0 ? t.n : t.zcount[zone];
+  if (n <= 0) return NPBMZ_OK;
+  int grid = n;
+  if (zone < 0 && c.solve_grid[DIR] > 0) grid = std::min(n, c.solve_grid[DIR]);
+  hipLaunchKernelGGL((fast::sp::solve_staged_kernel<DIR, FUSE>), dim3(grid), dim3(64),
+                     staged_lds(c.maxrows[DIR] + 2), c.stream, c.u, c.rhs, c.zd, t.d + first,
+                     n, c.maxrows[DIR] + 2, c.K, xraw);
+  CK(hipGetLastError());
+  return NPBMZ_OK;
+}
+
 template <int DIR, bool FUSE>
 int k_solve_t(npbmz_ctx* ctx, int zone, double* xraw = nullptr) {
   auto& c = *ctx;
@@ -758,6 +819,8 @@ int k_solve_t(npbmz_ctx* ctx, int zone, double* xraw = nullptr) {
   };
   if (c.bench == NPBMZ_SP) {
     if (strict(ctx)) go_sp(exact::sp::solve_kernel<DIR, FUSE>, kLineNT);
+    else if (((c.solve_twist >> DIR) & 1) && c.sp_staged[DIR])
+      return k_solve_staged<DIR, FUSE>(ctx, zone, xraw);
     else if (((c.solve_twist >> DIR) & 1) && c.sp_twist_ok[DIR])
       go_sp(fast::sp::solve_twist_kernel<DIR, FUSE>, 2 * kLineNT);
     else go_sp(fast::sp::solve_kernel<DIR, FUSE>, kLineNT);
@@ -1279,7 +1342,13 @@ int k_sp_adj_solve(npbmz_ctx* ctx, const double* us, const double* x, const doub
   if (t.n <= 0) return NPBMZ_OK;
   int grid = t.n;
   if (c.solve_grid[DIR] > 0) grid = std::min(t.n, c.solve_grid[DIR]);
-  if (((c.solve_twist >> DIR) & 1) && c.sp_twist_ok[DIR])
+  if (((c.solve_twist >> DIR) & 1) && c.sp_staged[DIR]) {
+    const Table& ts = c.t_row[DIR];
+    const int nl = c.maxrows[DIR] + 2;
+    const int gs = c.solve_grid[DIR] > 0 ? std::min(ts.n, c.solve_grid[DIR]) : ts.n;
+    hipLaunchKernelGGL(fast::sp::adj_solve_staged_kernel<DIR>, dim3(gs), dim3(64), staged_lds(nl),
+                       c.stream, us, x, gin, lam, ubar, c.zd, ts.d, ts.n, nl, c.K);
+  } else if (((c.solve_twist >> DIR) & 1) && c.sp_twist_ok[DIR])
     hipLaunchKernelGGL(fast::sp::adj_solve_twist_kernel<DIR>, dim3(grid), dim3(2 * kLineNT), 0,
                        c.stream, us, x, gin, lam, ubar, c.cscr, c.zd, t.d, t.n, c.maxrows[DIR],
                        c.K);
@@ -1723,6 +1792,7 @@ int npbmz_create(const npbmz_problem* p, int32_t flags, npbmz_ctx** out) {
   CKC(hipMemset(c.u, 0, fb));
   CKC(hipMemset(c.frc, 0, fb));
   CKC(hipMemset(c.rhs, 0, fb));
+  if (c.bench == NPBMZ_SP && !strict(ctx)) choose_staged(c);
   if ((rc = build_tables(ctx))) return bad(rc);
   if (c.bench == NPBMZ_LU) {
     // the zone and tile sweeps' LDS: the device's per-workgroup maximum, granted to
@@ -1782,16 +1852,18 @@ int npbmz_create(const npbmz_problem* p, int32_t flags, npbmz_ctx** out) {
     c.solve_rows = 7;
   }
   if (c.bench == NPBMZ_SP) {
-    // default: two-sided solves in the directions with fewer line tasks
-    // than the chip has CUs, as measured on MI355X (class A, at most 225
-    // tasks per direction: 0.112 -> 0.096 ms/step; class B, 360 to 864
-    // tasks: 0.203 -> 0.209, so one wave per 64 lines there)
+    // default: two-sided solves wherever the lines fit the staged form
+    // (ms/step against the one-wave and two-wave solves before it: class A
+    // 0.085 -> 0.054, class B 0.200 -> 0.141); otherwise the two-wave solve
+    // in the directions with fewer line tasks than the chip has CUs (class
+    // A, at most 225 tasks per direction: 0.112 -> 0.096 ms/step; class B,
+    // 360 to 864 tasks: 0.203 -> 0.209, so one wave per 64 lines there)
     int dev = 0, cus = 256;
     if (hipGetDevice(&dev) == hipSuccess)
       (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
     c.solve_twist = 0;
     for (int d = 0; d < 3; ++d)
-      if (c.sp_twist_ok[d] && c.t_line[d].n < cus) c.solve_twist |= 1 << d;
+      if (c.sp_twist_ok[d] && (c.sp_staged[d] || c.t_line[d].n < cus)) c.solve_twist |= 1 << d;
   }
   describe(ctx);
 #undef CKC
