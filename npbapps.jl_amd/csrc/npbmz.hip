@@ -13,7 +13,9 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <memory>
 #include <mutex>
+#include <new>
 #include <numeric>
 #include <string>
 #include <type_traits>
@@ -1933,28 +1935,47 @@ static int transfer(npbmz_ctx* ctx, int32_t zone, int32_t field, double* host,
   if ((rc = host_map(ctx, zone, lo, hi, order, dims))) return rc;
   const ZoneDev Z = ctx->zh[zone];
   const int origin = ctx->bench == NPBMZ_LU ? 1 : 0;
-  const size_t npt = (size_t)Z.nx * Z.ny * Z.nz;
-  std::vector<double> stage(npt * 5);
+  const size_t nd = (size_t)Z.nx * Z.ny * Z.nz * 5;
   double* dev = f + Z.base * 5;
-  if (!put) CK(hipMemcpyAsync(stage.data(), dev, stage.size() * sizeof(double),
-                              hipMemcpyDeviceToHost, ctx->stream));
+  // a host array of the zone's own shape and order is the zone's block of HBM
+  if (order == NPBMZ_ORDER_MIJK && dims[0] == 5 && dims[1] == Z.nx && dims[2] == Z.ny &&
+      dims[3] == Z.nz) {
+    CK(hipMemcpyAsync(put ? dev : host, put ? host : dev, nd * sizeof(double),
+                      put ? hipMemcpyHostToDevice : hipMemcpyDeviceToHost, ctx->stream));
+    CK(hipStreamSynchronize(ctx->stream));
+    return NPBMZ_OK;
+  }
+  std::unique_ptr<double[]> stage(new (std::nothrow) double[nd]);
+  if (!stage) return fail(ctx, NPBMZ_ENOMEM, "host staging");
+  if (!put) CK(hipMemcpyAsync(stage.get(), dev, nd * sizeof(double), hipMemcpyDeviceToHost,
+                              ctx->stream));
   if (!put) CK(hipStreamSynchronize(ctx->stream));
+  const int64_t si = order == NPBMZ_ORDER_MIJK ? dims[0] : 1;
+  const int64_t sm = order == NPBMZ_ORDER_MIJK ? 1 : dims[0] * dims[1] * dims[2];
+  const int64_t sj = si * dims[order == NPBMZ_ORDER_MIJK ? 1 : 0];
+  const int64_t sk = sj * dims[order == NPBMZ_ORDER_MIJK ? 2 : 1];
+  const int am = order == NPBMZ_ORDER_MIJK ? 0 : 3, ai = order == NPBMZ_ORDER_MIJK ? 1 : 0;
+  double* const org = host + (1 - lo[am]) * sm + (origin - lo[ai]) * si +
+                      (origin - lo[ai + 1]) * sj + (origin - lo[ai + 2]) * sk;
+  double* s = stage.get();
   for (int k = 0; k < Z.nz; ++k)
-    for (int j = 0; j < Z.ny; ++j)
-      for (int i = 0; i < Z.nx; ++i)
-        for (int m = 0; m < 5; ++m) {
-          int64_t ii = i + origin, jj = j + origin, kk = k + origin, mm = m + 1;
-          int64_t off;
-          if (order == NPBMZ_ORDER_MIJK)
-            off = (mm - lo[0]) + dims[0] * ((ii - lo[1]) + dims[1] * ((jj - lo[2]) + dims[2] * (kk - lo[3])));
-          else
-            off = (ii - lo[0]) + dims[0] * ((jj - lo[1]) + dims[1] * ((kk - lo[2]) + dims[2] * (mm - lo[3])));
-          size_t s = ((size_t)(k * Z.ny + j) * Z.nx + i) * 5 + m;
-          if (put) stage[s] = host[off];
-          else host[off] = stage[s];
+    for (int j = 0; j < Z.ny; ++j) {
+      double* h = org + j * sj + k * sk;
+      if (si == 5 && sm == 1) {  // the components of a row's points side by side
+        const size_t row = (size_t)Z.nx * 5 * sizeof(double);
+        if (put) std::memcpy(s, h, row);
+        else std::memcpy(h, s, row);
+        s += (size_t)Z.nx * 5;
+        continue;
+      }
+      for (int i = 0; i < Z.nx; ++i, h += si)
+        for (int m = 0; m < 5; ++m, ++s) {
+          if (put) *s = h[m * sm];
+          else h[m * sm] = *s;
         }
+    }
   if (put) {
-    CK(hipMemcpyAsync(dev, stage.data(), stage.size() * sizeof(double), hipMemcpyHostToDevice,
+    CK(hipMemcpyAsync(dev, stage.get(), nd * sizeof(double), hipMemcpyHostToDevice,
                       ctx->stream));
     CK(hipStreamSynchronize(ctx->stream));
   }
@@ -2483,27 +2504,33 @@ int npbmz_adjoint(npbmz_ctx* ctx, int32_t nsteps, int32_t ckpt_every, const doub
   // segment the post-exchange u and the three solve outputs (SP: also r0;
   // LU: the pre-exchange u in x3 and the sweep outputs in x1, x2, with one
   // more workspace field)
-  std::vector<double*> bufs;
-  auto alloc = [&](double** p) -> bool {
-    if (hipMalloc(p, fb) != hipSuccess) return false;
-    bufs.push_back(*p);
-    return true;
+  // in one allocation (of class A's 111 fields of 10 MB, one call each way took 25 ms)
+  const size_t nf = 4 + (lu || sp ? 2 : 0) + (size_t)ncp + (size_t)k * (sp ? 5 : 4);
+  const size_t field = (fb + 255) / 256 * 256;
+  char *arena = nullptr, *next = nullptr;
+  if (nf > SIZE_MAX / field || hipMalloc(&arena, nf * field) != hipSuccess) {
+    (void)hipGetLastError();
+    return fail(ctx, NPBMZ_ENOMEM, "adjoint buffers");
+  }
+  next = arena;
+  auto take = [&]() {
+    double* p = reinterpret_cast<double*>(next);
+    next += field;
+    return p;
   };
-  auto release = [&]() {
-    for (double* p : bufs) (void)hipFree(p);
-  };
-  double *wd, *ubar, *lam, *fbar, *aux = nullptr, *rs0 = nullptr;
-  std::vector<double*> ck(ncp), us(k), x1(k), x2(k), x3(k), r0(k, nullptr);
+  auto release = [&]() { (void)hipFree(arena); };
+  double *wd = take(), *ubar = take(), *lam = take(), *fbar = take();
   // LU: a workspace field and the saved rsd; SP: the y and x transposed
   // solutions (lam holds z's)
-  bool ok = alloc(&wd) && alloc(&ubar) && alloc(&lam) && alloc(&fbar) &&
-            (!(lu || sp) || (alloc(&aux) && alloc(&rs0)));
-  for (int q = 0; q < ncp && ok; ++q) ok = alloc(&ck[q]);
-  for (int q = 0; q < k && ok; ++q) ok = alloc(&us[q]) && alloc(&x1[q]) && alloc(&x2[q]) && alloc(&x3[q]);
-  for (int q = 0; q < k && ok && sp; ++q) ok = alloc(&r0[q]);
-  if (!ok) {
-    release();
-    return fail(ctx, NPBMZ_ENOMEM, "adjoint buffers");
+  double *aux = lu || sp ? take() : nullptr, *rs0 = lu || sp ? take() : nullptr;
+  std::vector<double*> ck(ncp), us(k), x1(k), x2(k), x3(k), r0(k, nullptr);
+  for (auto& p : ck) p = take();
+  for (int q = 0; q < k; ++q) {
+    us[q] = take();
+    x1[q] = take();
+    x2[q] = take();
+    x3[q] = take();
+    if (sp) r0[q] = take();
   }
   int rc = NPBMZ_OK;
   auto hip = [&](hipError_t e, const char* what) {

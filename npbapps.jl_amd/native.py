@@ -206,7 +206,16 @@ class Context:
 
     def get_all(self, field):
         """Every zone's field, zone after zone, each (nz, ny, nx, 5) flattened."""
-        return np.concatenate([self.get_dense(z, field).ravel() for z in range(self.zones.count)])
+        out = np.empty(self.size)
+        org = 1 if self.bench == LU else 0
+        off = 0
+        for z in range(self.zones.count):
+            n = [int(self.zones.nx[z]), int(self.zones.ny[z]), int(self.zones.nz[z])]
+            end = off + 5 * n[0] * n[1] * n[2]
+            self.get_field(z, field, out[off:end], (1, org, org, org),
+                           (5, n[0] - 1 + org, n[1] - 1 + org, n[2] - 1 + org))
+            off = end
+        return out
 
     def put_all(self, field, flat):
         flat = np.ascontiguousarray(flat, dtype=np.float64)
