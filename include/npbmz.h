@@ -235,7 +235,8 @@ int npbmz_tune(npbmz_ctx* ctx, int32_t budget_ms);
                                     block rows on five lanes, two-sided, keeping
                                     the last reduced rows of each half in
                                     registers (overrides TWIST and PAIR).
-                                    Default: all three directions (7) */
+                                    Default: all three directions (7), under
+                                    COLS */
 #define NPBMZ_SCHED_LU_TILES 7 /* LU pipelined sweep: tiles per zone, 1..8 (default:
                                   the padded slots over 256, rounded up, at most 8;
                                   4 where the tiles are not the default; fewer if a
@@ -267,6 +268,12 @@ int npbmz_tune(npbmz_ctx* ctx, int32_t budget_ms);
                                    exchange's blocks fill the halos for the line
                                    solves; same bits); 0 a launch of its own;
                                    default 1 */
+#define NPBMZ_SCHED_SOLVE_COLS 12 /* BT, FMA arithmetic only (ignored with
+                                     NPBMZ_FLAG_STRICT_FP): bit d set: direction d
+                                     solves five lines a wave, both halves of each
+                                     with the blocks' columns on six lanes
+                                     (overrides ROWS).  Default: all three
+                                     directions (7); setting ROWS sets it to 0 */
 int npbmz_set_schedule(npbmz_ctx* ctx, int32_t which, int32_t value);
 
 /* Describe the schedule currently in use (for logs); writes a NUL-terminated

@@ -144,6 +144,7 @@ __device__ __forceinline__ double recip(double x) {
 }
 #include "bt_kernels.inc"
 #include "bt_rows.inc"
+#include "bt_cols.inc"
 #include "bt_adjoint.inc"
 #include "sp_kernels.inc"
 #include "sp_lines.inc"
@@ -220,6 +221,11 @@ constexpr int kRowR = 6;     // reduced rows per half line kept in registers (ro
 constexpr int kRowRLong = 8; // the same where a direction's tasks need more than one round of
                              // waves: the rows kernel with its block rows read as applied
                              // (fewer registers live), less spill traffic
+// The columns kernel's reduced rows: per half line in registers (4 fill the
+// 256 VGPRs of two waves per SIMD; 3 and 5 are within 2%, 6 spills), and in
+// LDS (7 let eight waves share a CU; 6 cost class C 4%, none class B 5-10%).
+constexpr int kColR = 4;
+constexpr int kColLds = 7;
 constexpr int kPlaneNT = 64; // threads per block of an LU hyperplane launch
 constexpr int kGraphGroup = 8; // timesteps per replay of the grouped graph
 constexpr int kMaxSolveGrid = 65536; // largest persistent solve grid accepted
@@ -264,6 +270,7 @@ struct npbmz_ctx {
   int solve_twist = 7;            // BT/SP, FMA only: bit d set: solve_twist_kernel (wins over pair)
   bool sp_twist_ok[3] = {false, false, false};  // SP: every line of direction d has >= 4 unknowns
   int solve_rows = 0;             // BT, FMA only: bit d set: solve_rows_kernel (wins over twist);
+  int solve_cols = 0;             // BT, FMA only: bit d set: solve_cols_kernel (wins over rows)
   int cus = 256;                  // the device's compute units
                                   // set at creation by size
   int halfmax[3] = {0, 0, 0};     // rows of the longer half of the longest line per direction
@@ -287,6 +294,7 @@ struct npbmz_ctx {
   Table t_int, t_all, t_line[3], t_face, t_face2;
   Table t_row[3];  // BT: tasks of fast::bt::kRowLines lines for solve_rows_kernel; SP: of
                    // the staged solve's lines
+  Table t_col[3];  // BT: tasks of fast::bt::kColLines lines for solve_cols_kernel
   bool sp_staged[3] = {false, false, false};  // SP, FMA only: the direction's lines fit
                                               // solve_staged_kernel
   HaloSrc* hsrc = nullptr;  // BT/SP: where each zone side's halo cells come from
@@ -482,6 +490,28 @@ int lines_of(const npbmz_ctx* c, int z, int dir) {
 // tasks of `per` items.  The new device table is allocated before the old
 // one is freed, and t changes only on success, so a failure leaves the
 // previous table in place and usable.
+// solve_cols_kernel's reduced rows for half lines of at most halfmax rows:
+// the last kColR of a half in registers (none of a half shorter than that),
+// up to kColLds in LDS, the rest spilled.
+int cols_outside(int halfmax) { return std::max(halfmax - kColR, std::min(halfmax, kColR - 1)); }
+int cols_lds_rows(int halfmax) { return std::min(kColLds, cols_outside(halfmax)); }
+int cols_spill(int halfmax) { return cols_outside(halfmax) - cols_lds_rows(halfmax); }
+
+fast::bt::ColK make_col_constants(const StencilK& K, int d) {
+  fast::bt::ColK k{};
+  const double a1 = K.dt * K.t1[d];
+  k.ia = 1.0 / (K.dt * K.t2[d]);
+  k.c1 = K.c1;
+  k.c2 = K.c2;
+  k.k0 = a1 * k.ia * K.c3c4;
+  k.kd = K.con43 * k.k0;
+  k.k5 = a1 * k.ia * K.c1345;
+  k.kk0 = k.k0 - k.k5;
+  k.kkd = k.kd - k.k0;
+  for (int m = 0; m < 5; ++m) k.add[m] = a1 * k.ia * K.dd[d][m];
+  return k;
+}
+
 template <class F>
 int build_table(npbmz_ctx* ctx, Table& t, const std::vector<int>& order, int per, F count) {
   std::vector<Task> h;
@@ -566,6 +596,11 @@ int build_tables(npbmz_ctx* ctx) {
       c.halfmax[d] = (mr + 1) / 2;
       const size_t spill_rows = (size_t)std::max(0, c.halfmax[d] - kRowR);
       slot = std::max(slot, (size_t)c.t_row[d].n * spill_rows * 2 * 6 * 64);
+      // the columns kernel alike
+      if ((rc = build_table(ctx, c.t_col[d], ord, fast::bt::kColLines,
+                            [&](int z) { return lines_of(ctx, z, d); })))
+        return rc;
+      slot = std::max(slot, (size_t)c.t_col[d].n * cols_spill(c.halfmax[d]) * fast::bt::kColRow);
     } else if (c.sp_staged[d]) {
       if ((rc = build_table(ctx, c.t_row[d], ord, fast::sp::kStageLines,
                             [&](int z) { return lines_of(ctx, z, d); })))
@@ -826,6 +861,18 @@ int k_solve_t(npbmz_ctx* ctx, int zone, double* xraw = nullptr) {
     else if (((c.solve_twist >> DIR) & 1) && c.sp_twist_ok[DIR])
       go_sp(fast::sp::solve_twist_kernel<DIR, FUSE>, 2 * kLineNT);
     else go_sp(fast::sp::solve_kernel<DIR, FUSE>, kLineNT);
+  } else if (!strict(ctx) && ((c.solve_cols >> DIR) & 1)) {
+    const Table& tc = c.t_col[DIR];
+    const int f0 = zone < 0 ? 0 : tc.zfirst[zone], nr = zone < 0 ? tc.n : tc.zcount[zone];
+    if (nr <= 0) return NPBMZ_OK;
+    int gr = nr;
+    if (zone < 0 && c.solve_grid[DIR] > 0) gr = std::min(nr, c.solve_grid[DIR]);
+    const int lrows = cols_lds_rows(c.halfmax[DIR]);
+    const size_t lds = sizeof(double) * (2 * fast::bt::kColLines * fast::bt::kColSlot +
+                                         (size_t)lrows * fast::bt::kColRow);
+    hipLaunchKernelGGL((fast::bt::solve_cols_kernel<DIR, FUSE, kColR>), dim3(gr), dim3(64), lds,
+                       c.stream, c.u, c.rhs, c.cscr, c.zd, tc.d + f0, nr, lrows,
+                       cols_spill(c.halfmax[DIR]), make_col_constants(c.K, DIR));
   } else if (!strict(ctx) && ((c.solve_rows >> DIR) & 1)) {
     const Table& tr = c.t_row[DIR];
     const int f0 = zone < 0 ? 0 : tr.zfirst[zone], nr = zone < 0 ? tr.n : tr.zcount[zone];
@@ -1640,10 +1687,11 @@ void describe(npbmz_ctx* c) {
     for (int d = 0; d < 3; ++d)
       ring[d] = strict(c) || !((c->solve_rows >> d) & 1) ? 0 : rows_long(*c, d) ? kRowRLong : kRowR;
     snprintf(b, sizeof b,
-             "zones=%d order=%s solve_grid=%d/%d/%d pair=%d twist=%d rows=%d ring=%d/%d/%d fp=%s",
+             "zones=%d order=%s solve_grid=%d/%d/%d pair=%d twist=%d rows=%d ring=%d/%d/%d cols=%d fp=%s",
              c->nz_, c->largest_first ? "largest-first" : "natural", c->solve_grid[0],
              c->solve_grid[1], c->solve_grid[2], c->solve_pair, strict(c) ? 0 : c->solve_twist,
-             strict(c) ? 0 : c->solve_rows, ring[0], ring[1], ring[2], strict(c) ? "strict" : "fma");
+             strict(c) ? 0 : c->solve_rows, ring[0], ring[1], ring[2],
+             strict(c) ? 0 : c->solve_cols, strict(c) ? "strict" : "fma");
   }
   c->sched = b;
 }
@@ -1852,6 +1900,10 @@ int npbmz_create(const npbmz_problem* p, int32_t flags, npbmz_ctx** out) {
     // class S 0.057 / 0.039 / 0.037, W 0.083 / 0.056 / 0.054, A 0.172 /
     // 0.120 / 0.120, B 0.397 / 0.304 / 0.296, C 1.421 / 1.243 / 1.236
     c.solve_rows = 7;
+    // and over it the columns kernel, which is faster in every direction (us
+    // for the three solves of a step, rows / columns: class S 29.2 / 21.0, B
+    // 276 / 233, C 1055 / 902; 122 / 104 on 131x97x23 in 3x2 zones)
+    c.solve_cols = 7;
   }
   if (c.bench == NPBMZ_SP) {
     // default: two-sided solves wherever the lines fit the staged form
@@ -2294,6 +2346,8 @@ int npbmz_tune(npbmz_ctx* ctx, int32_t budget_ms) {
     if (!strict(ctx)) knobs.push_back({NPBMZ_SCHED_SOLVE_TWIST, {0, 1, 3, 7}});
     if (c.bench == NPBMZ_BT && !strict(ctx))
       knobs.push_back({NPBMZ_SCHED_SOLVE_ROWS, {0, 1, 3, 7}});
+    if (c.bench == NPBMZ_BT && !strict(ctx))  // after ROWS, which sets it to 0
+      knobs.push_back({NPBMZ_SCHED_SOLVE_COLS, {0, 1, 3, 7}});
     knobs.push_back({NPBMZ_SCHED_SOLVE_GRID, {0, 1024}});
     knobs.push_back({NPBMZ_SCHED_RHS_EXCH, {1, 0}});
   }
@@ -2307,6 +2361,7 @@ int npbmz_tune(npbmz_ctx* ctx, int32_t budget_ms) {
       case NPBMZ_SCHED_SOLVE_PAIR: return c.solve_pair;
       case NPBMZ_SCHED_SOLVE_TWIST: return c.solve_twist;
       case NPBMZ_SCHED_SOLVE_ROWS: return c.solve_rows;
+      case NPBMZ_SCHED_SOLVE_COLS: return c.solve_cols;
       case NPBMZ_SCHED_SOLVE_GRID: return c.solve_grid[0];
       case NPBMZ_SCHED_RHS_EXCH: return c.rhs_exch;
       default: return c.largest_first ? 1 : 0;
@@ -2441,6 +2496,12 @@ int npbmz_set_schedule(npbmz_ctx* ctx, int32_t which, int32_t value) {
       if (c.bench != NPBMZ_BT || value < 0 || value > 7)
         return fail(ctx, NPBMZ_EINVAL, "BT rows-over-lanes solve mask is 0..7");
       c.solve_rows = value;
+      c.solve_cols = 0;  // the rows kernel, or what it gives way to, as asked
+      break;
+    case NPBMZ_SCHED_SOLVE_COLS:
+      if (c.bench != NPBMZ_BT || value < 0 || value > 7)
+        return fail(ctx, NPBMZ_EINVAL, "BT columns solve mask is 0..7");
+      c.solve_cols = value;
       break;
     case NPBMZ_SCHED_RHS_EXCH:
       if (c.bench == NPBMZ_LU || value < 0 || value > 1)

@@ -30,6 +30,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
 # the sources whose text determines the BT kernels' memory traffic
 KERNEL_SOURCES = ("csrc/npbmz.hip", "csrc/bt_kernels.inc", "csrc/bt_rows.inc",
+                  "csrc/bt_cols.inc",
                   "csrc/npbmz_types.h")
 COPY_KERNEL = "copy_probe_kernel"
 # phase name (bench.py) -> pattern of the kernel that runs the phase (any of
