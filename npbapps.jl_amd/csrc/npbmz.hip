@@ -496,6 +496,10 @@ int lines_of(const npbmz_ctx* c, int z, int dir) {
 int cols_outside(int halfmax) { return std::max(halfmax - kColR, std::min(halfmax, kColR - 1)); }
 int cols_lds_rows(int halfmax) { return std::min(kColLds, cols_outside(halfmax)); }
 int cols_spill(int halfmax) { return cols_outside(halfmax) - cols_lds_rows(halfmax); }
+size_t cols_lds(int halfmax) {
+  return sizeof(double) * (2 * fast::bt::kColLines * fast::bt::kColSlot +
+                           (size_t)cols_lds_rows(halfmax) * fast::bt::kColRow);
+}
 
 fast::bt::ColK make_col_constants(const StencilK& K, int d) {
   fast::bt::ColK k{};
@@ -867,12 +871,10 @@ int k_solve_t(npbmz_ctx* ctx, int zone, double* xraw = nullptr) {
     if (nr <= 0) return NPBMZ_OK;
     int gr = nr;
     if (zone < 0 && c.solve_grid[DIR] > 0) gr = std::min(nr, c.solve_grid[DIR]);
-    const int lrows = cols_lds_rows(c.halfmax[DIR]);
-    const size_t lds = sizeof(double) * (2 * fast::bt::kColLines * fast::bt::kColSlot +
-                                         (size_t)lrows * fast::bt::kColRow);
-    hipLaunchKernelGGL((fast::bt::solve_cols_kernel<DIR, FUSE, kColR>), dim3(gr), dim3(64), lds,
-                       c.stream, c.u, c.rhs, c.cscr, c.zd, tc.d + f0, nr, lrows,
-                       cols_spill(c.halfmax[DIR]), make_col_constants(c.K, DIR));
+    hipLaunchKernelGGL((fast::bt::solve_cols_kernel<DIR, FUSE, kColR>), dim3(gr), dim3(64),
+                       cols_lds(c.halfmax[DIR]), c.stream, c.u, c.rhs, c.cscr, c.zd, tc.d + f0, nr,
+                       cols_lds_rows(c.halfmax[DIR]), cols_spill(c.halfmax[DIR]),
+                       make_col_constants(c.K, DIR));
   } else if (!strict(ctx) && ((c.solve_rows >> DIR) & 1)) {
     const Table& tr = c.t_row[DIR];
     const int f0 = zone < 0 ? 0 : tr.zfirst[zone], nr = zone < 0 ? tr.n : tr.zcount[zone];
@@ -1325,7 +1327,14 @@ int k_adj_solve(npbmz_ctx* ctx, const double* us, const double* x, const double*
   if (t.n <= 0) return NPBMZ_OK;
   int grid = t.n;
   if (c.solve_grid[DIR] > 0) grid = std::min(t.n, c.solve_grid[DIR]);
-  if ((c.solve_twist >> DIR) & 1)
+  if ((c.solve_cols >> DIR) & 1) {
+    const Table& tc = c.t_col[DIR];
+    const int gc = c.solve_grid[DIR] > 0 ? std::min(tc.n, c.solve_grid[DIR]) : tc.n;
+    hipLaunchKernelGGL((fast::bt::adj_solve_cols_kernel<DIR, kColR>), dim3(gc), dim3(64),
+                       cols_lds(c.halfmax[DIR]), c.stream, us, gin, lam, c.cscr, c.zd, tc.d, tc.n,
+                       cols_lds_rows(c.halfmax[DIR]), cols_spill(c.halfmax[DIR]),
+                       make_col_constants(c.K, DIR));
+  } else if ((c.solve_twist >> DIR) & 1)
     hipLaunchKernelGGL(fast::bt::adj_solve_twist_kernel<DIR>, dim3(grid), dim3(2 * kLineNT), 0,
                        c.stream, us, gin, lam, c.cscr, c.zd, t.d, t.n, c.maxrows[DIR], c.K);
   else

@@ -81,3 +81,30 @@ def test_columns_knob_is_validated_and_rows_replaces_it(gpu):
     with pytest.raises(gpu.NpbmzError):
         ctx.set_schedule(N.SCHED_SOLVE_COLS, 7)
     ctx.close()
+
+
+@pytest.mark.parametrize("grid,zones,ratio", GRIDS)
+def test_columns_adjoint_tracks_the_two_sided_one(gpu, grid, zones, ratio):
+    """Gradients of a weighted sum of squares through three steps, forward
+    and transposed solves by columns against both two-sided: 1e-12 of the
+    gradient's size, a hundred times the forward's bound for the
+    cancellations of the reverse pass."""
+    N = gpu.native
+    out = []
+    for cols, size in ((0, 0), (7, 0), (7, 3)):
+        ctx = gpu.Context("BT", gpu.zone_setup(*zones, *grid, ratio), 0.0003)
+        ctx.set_schedule(N.SCHED_SOLVE_ROWS, 0)
+        ctx.set_schedule(N.SCHED_SOLVE_COLS, cols)
+        ctx.set_schedule(N.SCHED_SOLVE_GRID, size)
+        ctx.init_exact()
+        u = ctx.get_all(0)
+        rng = np.random.default_rng(5)
+        ctx.put_all(0, u * (1.0 + 0.02 * rng.uniform(-1.0, 1.0, u.size)))
+        out.append(ctx.adjoint(3, 2, np.random.default_rng(3).random(ctx.size)))
+        ctx.close()
+    a, b, c = out
+    assert abs(b["loss"] / a["loss"] - 1.0) <= 1e-13
+    for k in ("grad_u0", "grad_forcing"):
+        assert np.isfinite(a[k]).all()
+        assert np.abs(a[k] - b[k]).max() <= 1e-12 * np.abs(a[k]).max(), k
+        assert np.array_equal(b[k], c[k]), k
