@@ -237,11 +237,18 @@ enum { kSweepPlane = 0, kSweepZone = 1, kSweepTiles = 2 };
 constexpr int kMaxTiles = 8;    // tiles per zone of the pipelined sweep
 constexpr int kMaxGroups = 16;  // workgroups per zone its tiles may take
 
-// A task table on the device plus, per zone, the range of its tasks.
+// A task table on the device plus, per zone, the range of its tasks; freed
+// with the context that holds it.
 struct Table {
   Task* d = nullptr;
   int n = 0;
   std::vector<int> zfirst, zcount;  // by zone number
+  Table() = default;
+  Table(const Table&) = delete;
+  Table& operator=(const Table&) = delete;
+  ~Table() {
+    if (d) (void)hipFree(d);
+  }
 };
 
 }  // namespace
@@ -1939,10 +1946,6 @@ void npbmz_destroy(npbmz_ctx* ctx) {
   auto& c = *ctx;
   if (c.stream) (void)hipStreamSynchronize(c.stream);
   drop_graphs(c);
-  Table* ts[] = {&c.t_int,    &c.t_all,    &c.t_line[0], &c.t_line[1], &c.t_line[2],
-                 &c.t_face,   &c.t_face2,  &c.t_row[0],  &c.t_row[1],  &c.t_row[2]};
-  for (Table* t : ts)
-    if (t->d) (void)hipFree(t->d);
   void* ps[] = {c.zd, c.u, c.frc, c.rhs, c.cscr, c.faces, c.partial, c.zpart, c.txbuf, c.tcnt,
                 c.hsrc};
   for (void* q : ps)
