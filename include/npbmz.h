@@ -258,9 +258,10 @@ int npbmz_tune(npbmz_ctx* ctx, int32_t budget_ms);
                                      rows need no cache maintenance (the default where
                                      the device places workgroup b on the XCD of
                                      workgroup b mod 8, which is checked once per
-                                     device; EINVAL elsewhere); 2 as 1 with every tile's
-                                     placement check failing, for tests of the error
-                                     path (the step fails with NPBMZ_EHIP) */
+                                     device; EINVAL elsewhere); 2 as 1 with a zone's
+                                     tiles on different XCDs, for tests of the check
+                                     and its error path (the step fails with
+                                     NPBMZ_EHIP) */
 #define NPBMZ_SCHED_RHS_EXCH 11 /* BT and SP with more than one zone: 1 batched and
                                    graph steps run the zone-face exchange in
                                    compute_rhs's launch (the rhs reads each face

@@ -291,7 +291,7 @@ struct npbmz_ctx {
   int lu_kb = 4;                  // pipelined sweep: hyperplanes per published count
   int lu_spin = 1 << 20;          // pipelined sweep: polls before a wait gives up
   int lu_handoff = -1;            // pipelined sweep: 0 agent-scope, 1 XCD-local, 2 XCD-local
-                                  // with every placement check failing; -1 XCD-local where
+                                  // with tiles placed for its check to fail; -1 XCD-local where
                                   // it applies
   bool tile_local_ok = false;     // this device places blocks of equal b mod 8 on one XCD
   double* txbuf = nullptr;        // pipelined sweep: tile edge rows of every hyperplane
@@ -1105,8 +1105,8 @@ int check_tiles(npbmz_ctx* ctx) {
                       : "LU pipelined sweep: a tile's wait for its upstream tile exceeded its bound");
 }
 
-// The hand-off the pipelined sweep runs: XCD-local (1; 2 with a map that
-// no tile matches) or agent-scope (0).
+// The hand-off the pipelined sweep runs: XCD-local (1; 2 with each zone's
+// workgroups on different XCDs, which its check reports) or agent-scope (0).
 int tile_handoff(const npbmz_ctx* c) {
   if (c->lu_handoff >= 0) return c->lu_handoff;
   return c->tile_local_ok ? 1 : 0;
@@ -1132,14 +1132,14 @@ int k_lu_sweep_t(npbmz_ctx* ctx, int zone, bool* upd = nullptr) {
     int* const dn = cn + (size_t)c.nz_ * kMaxGroups;
     int* const ef = dn + c.nz_;
     // workgroup w of zone zl is block w * nzp + zl: the same residue mod 8 for
-    // all of a zone
-    const int nzp = (nzl + 7) & ~7;
+    // all of a zone (hand-off 2: one more from each to the next)
     const int ho = tile_handoff(&c);
+    const int nzp = ((nzl + 7) & ~7) + (ho == 2 ? 1 : 0);
     int* const xc = ef + 1;
     auto go = [&](auto kern) {
       hipLaunchKernelGGL(kern, dim3(nzp * g.G), dim3(g.nt + 64), g.lds, c.stream, c.u, c.rhs, c.zd,
                          z0, nzl, nzp, g.G, g.rpt, g.parts, c.lu_kb, g.steps, c.txbuf, cn, dn, ef, c.lu_spin,
-                         xc, ho == 2 ? 1 : 0, c.lk);
+                         xc, c.lk);
     };
     // the hand-off form: XCD-local with 4 or 8 doubles of a row per lane, or
     // agent-scope
@@ -2473,7 +2473,7 @@ int npbmz_set_schedule(npbmz_ctx* ctx, int32_t which, int32_t value) {
       if (c.bench != NPBMZ_LU || value < 0 || value > 2)
         return fail(ctx, NPBMZ_EINVAL,
                     "LU tile hand-off is 0 (agent scope), 1 (XCD-local) or 2 (XCD-local, "
-                    "placement check forced to fail)");
+                    "tiles placed for its check to fail)");
       {
         const int rc = ensure_tiles(ctx);
         if (rc) return rc;

@@ -10,6 +10,8 @@ for bit with them; runs track the oracle per iteration and verify.  Every
 wait between tiles is bounded: with the bound forced to fail, the step
 reports an error and the context stays usable.
 """
+import time
+
 import numpy as np
 import pytest
 
@@ -145,10 +147,9 @@ def test_handoffs_agree_bitwise(gpu, cls, tiles, batch):
 
 
 def test_handoff_placement_check_reports_an_error_and_recovers(gpu):
-    """Hand-off 2 runs the XCD-local kernel with a placement map that no
-    tile matches: every tile stops at its check, the step reports the
-    placement error, and with hand-off 1 the context runs a verified class W
-    run."""
+    """Hand-off 2 runs the XCD-local kernel with a zone's tiles on different
+    XCDs: every tile stops at its check, the step reports the placement
+    error, and with hand-off 1 the context runs a verified class W run."""
     N = gpu.native
     ctx, zones, p = _ctx(gpu, "W")
     ctx.set_schedule(N.SCHED_LU_HANDOFF, 2)
@@ -160,6 +161,23 @@ def test_handoff_placement_check_reports_an_error_and_recovers(gpu):
     ctx.step(p.niter, "graph")
     xcr, xce, xci = ctx.norms()
     assert gpu.verify.verify("LU", "W", p.dt, p.niter, xcr, xce, xci)[0]
+    ctx.close()
+
+
+@pytest.mark.parametrize("cls,mode", [("A", "graph"), ("B", "batched"), ("B", "perzone")])
+def test_tiles_off_their_zones_xcd_are_found_before_any_wait(gpu, cls, mode):
+    """Tiles really on different XCDs, several iterations queued: the error is
+    the placement one, not a wait that ran out its bound on counts that stayed
+    in another XCD's L2, and no wait costs time (a wait that runs out takes
+    some 0.5 s, and each sweep would have one)."""
+    N = gpu.native
+    ctx, zones, p = _ctx(gpu, cls)
+    ctx.set_schedule(N.SCHED_LU_HANDOFF, 2)
+    ctx.init_exact()
+    start = time.monotonic()
+    with pytest.raises(gpu.NpbmzError, match="XCD"):
+        ctx.step(4, mode)
+    assert time.monotonic() - start < 2.0
     ctx.close()
 
 
