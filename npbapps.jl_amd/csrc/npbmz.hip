@@ -1061,6 +1061,10 @@ bool xcd_round_robin() {
   return state[dev] == 1;
 }
 
+// The tile sweep's counters: per workgroup the finished hyperplanes, per zone
+// the workgroups done, the error flag, per workgroup its XCD plus one.
+size_t tile_counters(const npbmz_ctx* c) { return (size_t)c->nz_ * kMaxGroups * 2 + c->nz_ + 1; }
+
 // Exchange rows and counters of the tile sweep, allocated once per context
 // for up to kMaxGroups workgroups per zone, zeroed (each launch leaves them zero),
 // and the device's workgroup placement for the XCD-local hand-off.
@@ -1070,7 +1074,7 @@ int ensure_tiles(npbmz_ctx* ctx) {
   c.tile_local_ok = xcd_round_robin();
   const TileGeom g = tile_geom(&c);
   const size_t nx = (size_t)c.nz_ * kMaxGroups * g.steps * g.SJ * 5;
-  const size_t nc = (size_t)c.nz_ * kMaxGroups * 2 + c.nz_ + 1;
+  const size_t nc = tile_counters(&c);
   double* xb = nullptr;
   int* cn = nullptr;
   hipError_t e = hipMalloc(&xb, nx * sizeof(double));
@@ -1088,7 +1092,9 @@ int ensure_tiles(npbmz_ctx* ctx) {
 }
 
 // After work that may have run tile sweeps: a wait that hit its bound shows
-// as the error flag, which is reported and cleared.
+// as the error flag, which is reported.  The flag and every counter are
+// cleared with it: off its zone's XCD a workgroup's counts can reach memory
+// only at its kernel's end, after the zone's last one has reset them.
 int check_tiles(npbmz_ctx* ctx) {
   auto& c = *ctx;
   if (!c.tcnt) return NPBMZ_OK;
@@ -1097,8 +1103,7 @@ int check_tiles(npbmz_ctx* ctx) {
   CK(hipMemcpyAsync(&v, ef, sizeof v, hipMemcpyDeviceToHost, c.stream));
   CK(hipStreamSynchronize(c.stream));
   if (v == 0) return NPBMZ_OK;
-  const int zero = 0;
-  CK(hipMemcpyAsync(ef, &zero, sizeof zero, hipMemcpyHostToDevice, c.stream));
+  CK(hipMemsetAsync(c.tcnt, 0, tile_counters(&c) * sizeof(int), c.stream));
   CK(hipStreamSynchronize(c.stream));
   return fail(ctx, NPBMZ_EHIP,
               (v & 2) ? "LU pipelined sweep: a tile ran off its zone's XCD (XCD-local hand-off)"

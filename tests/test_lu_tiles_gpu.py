@@ -181,6 +181,31 @@ def test_tiles_off_their_zones_xcd_are_found_before_any_wait(gpu, cls, mode):
     ctx.close()
 
 
+@pytest.mark.parametrize("how", ["placement", "bound"])
+@pytest.mark.parametrize("handoff", [0, 1])
+def test_a_failed_sweep_leaves_no_counts_behind(gpu, how, handoff):
+    """After a step whose sweeps failed, at once and with more of them queued,
+    either hand-off gives the bits of a fresh context: no workgroup finds a
+    count of the failed sweeps and reads rows before they are written."""
+    N = gpu.native
+    out = []
+    for fail_first in (False, True):
+        ctx, zones, p = _ctx(gpu, "B", tiles=8)
+        if fail_first:
+            ctx.set_schedule(N.SCHED_LU_HANDOFF, 2 if how == "placement" else 1)
+            ctx.set_schedule(N.SCHED_LU_SPIN, 1 << 20 if how == "placement" else -1)
+            ctx.init_exact()
+            with pytest.raises(gpu.NpbmzError, match="pipelined sweep"):
+                ctx.step(3, "batched")
+            ctx.set_schedule(N.SCHED_LU_SPIN, 1 << 20)
+        ctx.set_schedule(N.SCHED_LU_HANDOFF, handoff)
+        ctx.init_exact()
+        ctx.step(3, "batched")
+        out.append((ctx.get_all(0), ctx.get_all(2)))
+        ctx.close()
+    assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
+
+
 def test_tile_knobs_are_validated(gpu):
     N = gpu.native
     ctx, zones, p = _ctx(gpu, "S")
