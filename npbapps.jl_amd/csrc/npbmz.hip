@@ -23,6 +23,7 @@
 
 #include "../../include/npbmz.h"
 #include "npbmz_types.h"
+#include "sp_lines_index.h"
 
 namespace npbmz {
 
