@@ -208,13 +208,16 @@ int npbmz_tune(npbmz_ctx* ctx, int32_t budget_ms);
                                      in the middle (BT: two waves per 64 lines,
                                      overrides PAIR, default 7; SP: for directions
                                      whose lines all have >= 6 points, six lines a
-                                     wave staged in LDS, default on where six of the
-                                     direction's lines fit it, up to 310 points;
-                                     longer lines two waves per 64, default on where
-                                     the direction has fewer line tasks of 64
-                                     lines than the device has CUs); the
-                                     adjoint's transposed solves follow the
-                                     same bits */
+                                     wave staged in LDS where that is the faster
+                                     form (along x wherever six lines fit, up to 310
+                                     points; along y and z by how many waves their
+                                     LDS leaves on a CU and how many tasks there
+                                     are; npbmz_describe's staged=, forward and
+                                     transposed), else two waves per 64 lines.
+                                     Default: on where staged, and where the
+                                     direction has fewer line tasks of 64 lines than
+                                     the device has CUs); the adjoint's transposed
+                                     solves follow the same bits */
 #define NPBMZ_SCHED_LU_FORWARD 5 /* LU workgroup-per-zone sweeps: each hyperplane
                                     hands the next its new rsd (1), or its rsd and
                                     u (2), through LDS, as far as two hyperplanes

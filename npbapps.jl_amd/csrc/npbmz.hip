@@ -276,6 +276,7 @@ struct npbmz_ctx {
   // two-sided solve) the wave pair in y.
   int solve_pair = 2;             // BT: bit d set: direction d uses solve_pair_kernel
   int solve_twist = 7;            // BT/SP, FMA only: bit d set: solve_twist_kernel (wins over pair)
+  int adj_twist = 7;              // the same for the transposed solves; set together
   bool sp_twist_ok[3] = {false, false, false};  // SP: every line of direction d has >= 4 unknowns
   int solve_rows = 0;             // BT, FMA only: bit d set: solve_rows_kernel (wins over twist);
   int solve_cols = 0;             // BT, FMA only: bit d set: solve_cols_kernel (wins over rows)
@@ -303,8 +304,9 @@ struct npbmz_ctx {
   Table t_row[3];  // BT: tasks of fast::bt::kRowLines lines for solve_rows_kernel; SP: of
                    // the staged solve's lines
   Table t_col[3];  // BT: tasks of fast::bt::kColLines lines for solve_cols_kernel
-  bool sp_staged[3] = {false, false, false};  // SP, FMA only: the direction's lines fit
-                                              // solve_staged_kernel
+  // SP, FMA only: the directions that solve_staged_kernel and
+  // adj_solve_staged_kernel take
+  bool sp_staged[3] = {false, false, false}, sp_adj_staged[3] = {false, false, false};
   HaloSrc* hsrc = nullptr;  // BT/SP: where each zone side's halo cells come from
   bool hsrc_ok = false;     // hsrc describes the face table exactly
   int rhs_exch = 1;         // BT/SP batched steps: 1 exchange inside compute_rhs's launch
@@ -613,7 +615,7 @@ int build_tables(npbmz_ctx* ctx) {
                             [&](int z) { return lines_of(ctx, z, d); })))
         return rc;
       slot = std::max(slot, (size_t)c.t_col[d].n * cols_spill(c.halfmax[d]) * fast::bt::kColRow);
-    } else if (c.sp_staged[d]) {
+    } else if (c.sp_staged[d] || c.sp_adj_staged[d]) {
       if ((rc = build_table(ctx, c.t_row[d], ord, fast::sp::kStageLines,
                             [&](int z) { return lines_of(ctx, z, d); })))
         return rc;
@@ -802,8 +804,32 @@ bool rows_long(const npbmz_ctx& c, int d) {
   return c.t_row[d].n > 4 * c.cus && c.halfmax[d] > kRowRLong;
 }
 
+// Waves of SP's staged solve that a CU's LDS holds, for lines of at most nl
+// points; it is granted in 1280-byte pieces.
+int64_t staged_waves(int nl, int lds) {
+  const size_t piece = 1280;
+  return (int64_t)(lds / ((staged_lds(nl) + piece - 1) / piece * piece));
+}
+
 // Where SP runs the staged solve: lines of 6 points and more, six of which
-// fit a workgroup's LDS (up to 310 points in 160 KB).
+// fit a workgroup's LDS (up to 310 points in 160 KB), and there where it is
+// the faster one.  Along x it is, at any length.  Along y and z the other
+// kernels' lanes share cache lines, and what counts is w, the waves per CU
+// that the lines' LDS leaves (3 up to 102 points, 2 up to 155, then 1):
+//  - it takes about r L (0.16, 0.2, 0.21, 0.23 us for w = 1, 2, 3, 4) for
+//    lines of L points in r rounds of w waves per CU.  The two-wave solve,
+//    taken where it has fewer tasks than CUs, takes 0.6 to 0.7 L whatever
+//    their number, so the line is at 2 (w + 1) tasks per CU.  us along y, two
+//    waves and staged: 1 M points, L = 128 81 and 73, 160 98 and 100; 1.5 M, 96
+//    69 and 83, 128 83 and 97, 200 123 and 155; 2 M, 140 95 and 132, 300
+//    180 and 183;
+//  - against the one-wave solve, taken from there on, it loses with one wave
+//    per CU (8 M points along y and z, L = 170: 485 and 545 us, staged 833
+//    and 940) and is level or wins with two and more (128: 475 and 550,
+//    staged 493 and 564; 77: 470 and 547, staged 305 and 362).
+// The transposed kernels differ more: with w = 1 the line is at 5 tasks per
+// CU (y: 2 M points, L = 160 162 us, staged 245; 300 275 and 232), with w = 2
+// at 25 (L = 128: 4 M 299 and 281, 6 M 345 and 419, 12 M 649 and 820).
 void choose_staged(npbmz_ctx& c) {
   int dev = 0, lds = 0;
   if (hipGetDevice(&dev) != hipSuccess ||
@@ -827,9 +853,18 @@ void choose_staged(npbmz_ctx& c) {
   }
   for (int d = 0; d < 3; ++d) {
     int nl = 0;
-    for (int z = 0; z < c.nz_; ++z)
+    int64_t six = 0, wave = 0;  // tasks of the staged and of the other kernels
+    for (int z = 0; z < c.nz_; ++z) {
       nl = std::max(nl, d == 0 ? c.nx[z] : d == 1 ? c.ny[z] : c.nz[z]);
-    c.sp_staged[d] = c.sp_twist_ok[d] && staged_lds(nl) <= (size_t)lds;
+      const int n = lines_of(&c, z, d);
+      six += (n + fast::sp::kStageLines - 1) / fast::sp::kStageLines;
+      wave += (n + kLineNT - 1) / kLineNT;
+    }
+    const bool fits = c.sp_twist_ok[d] && staged_lds(nl) <= (size_t)lds;
+    const int64_t w = staged_waves(nl, lds);
+    c.sp_staged[d] =
+        fits && (d == 0 || six <= 2 * c.cus * (w + 1) || (w >= 2 && wave >= c.cus));
+    c.sp_adj_staged[d] = fits && (d == 0 || w >= 3 || six <= (w == 2 ? 25 : 5) * c.cus);
   }
 }
 
@@ -1347,7 +1382,7 @@ int k_adj_solve(npbmz_ctx* ctx, const double* us, const double* x, const double*
                        cols_lds(c.halfmax[DIR]), c.stream, us, gin, lam, c.cscr, c.zd, tc.d, tc.n,
                        cols_lds_rows(c.halfmax[DIR]), cols_spill(c.halfmax[DIR]),
                        make_col_constants(c.K, DIR));
-  } else if ((c.solve_twist >> DIR) & 1)
+  } else if ((c.adj_twist >> DIR) & 1)
     hipLaunchKernelGGL(fast::bt::adj_solve_twist_kernel<DIR>, dim3(grid), dim3(2 * kLineNT), 0,
                        c.stream, us, gin, lam, c.cscr, c.zd, t.d, t.n, c.maxrows[DIR], c.K);
   else
@@ -1413,13 +1448,13 @@ int k_sp_adj_solve(npbmz_ctx* ctx, const double* us, const double* x, const doub
   if (t.n <= 0) return NPBMZ_OK;
   int grid = t.n;
   if (c.solve_grid[DIR] > 0) grid = std::min(t.n, c.solve_grid[DIR]);
-  if (((c.solve_twist >> DIR) & 1) && c.sp_staged[DIR]) {
+  if (((c.adj_twist >> DIR) & 1) && c.sp_adj_staged[DIR]) {
     const Table& ts = c.t_row[DIR];
     const int nl = c.maxrows[DIR] + 2;
     const int gs = c.solve_grid[DIR] > 0 ? std::min(ts.n, c.solve_grid[DIR]) : ts.n;
     hipLaunchKernelGGL(fast::sp::adj_solve_staged_kernel<DIR>, dim3(gs), dim3(64), staged_lds(nl),
                        c.stream, us, x, gin, lam, ubar, c.zd, ts.d, ts.n, nl, c.K);
-  } else if (((c.solve_twist >> DIR) & 1) && c.sp_twist_ok[DIR])
+  } else if (((c.adj_twist >> DIR) & 1) && c.sp_twist_ok[DIR])
     hipLaunchKernelGGL(fast::sp::adj_solve_twist_kernel<DIR>, dim3(grid), dim3(2 * kLineNT), 0,
                        c.stream, us, x, gin, lam, ubar, c.cscr, c.zd, t.d, t.n, c.maxrows[DIR],
                        c.K);
@@ -1694,14 +1729,18 @@ void describe(npbmz_ctx* c) {
              : lu_fwd_level(c) == 1    ? " lds-forward=rsd"
                                        : "",
              (c->flags & NPBMZ_FLAG_LU_NPB_EXCH) ? "npb" : "reference", strict(c) ? "strict" : "fma");
-  else if (c->bench == NPBMZ_SP)
-    snprintf(b, sizeof b, "zones=%d order=%s solve_grid=%d/%d/%d twist=%d fp=%s", c->nz_,
+  else if (c->bench == NPBMZ_SP) {
+    int ok = 0, staged = 0, adj = 0;
+    for (int d = 0; d < 3; ++d) {
+      ok |= (!strict(c) && c->sp_twist_ok[d]) << d;
+      staged |= c->sp_staged[d] << d;
+      adj |= c->sp_adj_staged[d] << d;
+    }
+    snprintf(b, sizeof b, "zones=%d order=%s solve_grid=%d/%d/%d twist=%d staged=%d/%d fp=%s", c->nz_,
              c->largest_first ? "largest-first" : "natural", c->solve_grid[0],
-             c->solve_grid[1], c->solve_grid[2],
-             strict(c) ? 0
-                       : (c->solve_twist & ((c->sp_twist_ok[0] ? 1 : 0) | (c->sp_twist_ok[1] ? 2 : 0) |
-                                            (c->sp_twist_ok[2] ? 4 : 0))),
-             strict(c) ? "strict" : "fma");
+             c->solve_grid[1], c->solve_grid[2], c->solve_twist & ok, c->solve_twist & ok & staged,
+             c->adj_twist & ok & adj, strict(c) ? "strict" : "fma");
+  }
   else
   {
     // the rows kernel's ring of reduced rows per direction (0: not used)
@@ -1928,18 +1967,18 @@ int npbmz_create(const npbmz_problem* p, int32_t flags, npbmz_ctx** out) {
     c.solve_cols = 7;
   }
   if (c.bench == NPBMZ_SP) {
-    // default: two-sided solves wherever the lines fit the staged form
-    // (ms/step against the one-wave and two-wave solves before it: class A
-    // 0.085 -> 0.054, class B 0.200 -> 0.141); otherwise the two-wave solve
-    // in the directions with fewer line tasks than the chip has CUs (class
-    // A, at most 225 tasks per direction: 0.112 -> 0.096 ms/step; class B,
-    // 360 to 864 tasks: 0.203 -> 0.209, so one wave per 64 lines there)
-    int dev = 0, cus = 256;
-    if (hipGetDevice(&dev) == hipSuccess)
-      (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-    c.solve_twist = 0;
-    for (int d = 0; d < 3; ++d)
-      if (c.sp_twist_ok[d] && (c.sp_staged[d] || c.t_line[d].n < cus)) c.solve_twist |= 1 << d;
+    // default: two-sided solves wherever the staged form is taken (ms/step
+    // against the one-wave and two-wave solves: class A 0.085 -> 0.054,
+    // class B 0.200 -> 0.141); otherwise the two-wave solve in the directions
+    // with fewer line tasks than the chip has CUs (class A, at most 225 tasks
+    // per direction: 0.112 -> 0.096 ms/step; class B, 360 to 864 tasks: 0.203
+    // -> 0.209, so one wave per 64 lines there)
+    c.solve_twist = c.adj_twist = 0;
+    for (int d = 0; d < 3; ++d) {
+      if (!c.sp_twist_ok[d]) continue;
+      if (c.sp_staged[d] || c.t_line[d].n < c.cus) c.solve_twist |= 1 << d;
+      if (c.sp_adj_staged[d] || c.t_line[d].n < c.cus) c.adj_twist |= 1 << d;
+    }
   }
   describe(ctx);
 #undef CKC
@@ -2508,7 +2547,7 @@ int npbmz_set_schedule(npbmz_ctx* ctx, int32_t which, int32_t value) {
     case NPBMZ_SCHED_SOLVE_TWIST:
       if (c.bench == NPBMZ_LU || value < 0 || value > 7)
         return fail(ctx, NPBMZ_EINVAL, "BT/SP two-sided solve mask is 0..7");
-      c.solve_twist = value;
+      c.solve_twist = c.adj_twist = value;
       break;
     case NPBMZ_SCHED_SOLVE_ROWS:
       if (c.bench != NPBMZ_BT || value < 0 || value > 7)

@@ -1,14 +1,17 @@
 """SP's line solves staged in LDS: forward steps and gradients against the
 one-wave solves, at line counts that leave partial tasks, at the shortest
 lines the two-sided elimination takes, and at both sides of the longest that
-fit a workgroup's LDS (310 points; longer ones keep the two-wave solve)."""
+fit a workgroup's LDS (310 points; longer ones keep the two-wave solve).  And
+where they are taken: along y and z long lines leave few waves on a CU, and
+from some number of tasks on the other kernels are faster."""
 import numpy as np
 import pytest
 
 pytestmark = pytest.mark.gpu
 
 # (grid, zones, ratio): every direction's shortest lines; uneven odd zones;
-# the longest staged lines along x, y and z; lines too long to stage
+# the longest staged lines along x, y and z; lines too long to stage along
+# each; staged along x only, transposed in all three
 GRIDS = [
     ((6, 6, 6), (1, 1), 1.0),
     ((31, 25, 7), (2, 3), 1.6),
@@ -17,6 +20,9 @@ GRIDS = [
     ((8, 620, 6), (1, 2), 1.0),
     ((6, 7, 310), (1, 1), 1.0),
     ((311, 7, 6), (1, 1), 1.0),
+    ((6, 311, 7), (1, 1), 1.0),
+    ((7, 6, 311), (1, 1), 1.0),
+    ((84, 160, 84), (1, 1), 1.0),
 ]
 
 
@@ -68,3 +74,31 @@ def test_staged_adjoint_tracks_the_one_wave_one(gpu, grid, zones, ratio):
     for k in ("grad_u0", "grad_forcing"):
         assert np.isfinite(a[k]).all()
         assert np.abs(a[k] - b[k]).max() <= 1e-12 * np.abs(a[k]).max(), k
+
+
+# (grid, zones, ratio), the directions staged (bit d) forward and transposed:
+# the classes; long lines with few tasks; one wave per CU and over 4 tasks
+# each along y (1121), z's 3 waves and over 8 (2160); the same with over 5
+# along y and z; two waves and tasks over 25 per CU; lines too long
+ROUTES = [
+    ((128, 128, 16), (4, 4), 1.0, 7, 7),
+    ((304, 208, 17), (8, 8), 1.0, 7, 7),
+    ((310, 7, 6), (1, 1), 1.0, 7, 7),
+    ((6, 7, 310), (1, 1), 1.0, 7, 7),
+    ((84, 160, 84), (1, 1), 1.0, 1, 7),
+    ((100, 160, 160), (1, 1), 1.0, 1, 1),
+    ((160, 128, 160), (2, 2), 1.0, 3, 3),
+    ((140, 300, 140), (2, 2), 1.0, 7, 3),
+    ((6, 311, 7), (1, 1), 1.0, 5, 5),
+]
+
+
+@pytest.mark.parametrize("grid,zones,ratio,forward,transposed", ROUTES)
+def test_staged_where_it_is_the_faster_one(gpu, grid, zones, ratio, forward, transposed):
+    z = gpu.zone_setup(*zones, *grid, ratio)
+    ctx = gpu.Context("SP", z, 0.0007)
+    assert "staged=%d/%d" % (forward, transposed) in ctx.describe(), ctx.describe()
+    ctx.close()
+    ctx = gpu.Context("SP", z, 0.0007, strict=True)
+    assert "staged=0/0" in ctx.describe()
+    ctx.close()
