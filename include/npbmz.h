@@ -277,9 +277,11 @@ int npbmz_tune(npbmz_ctx* ctx, int32_t budget_ms);
                                      solves five lines a wave, both halves of each
                                      with the blocks' columns on six lanes
                                      (overrides ROWS); the adjoint's transposed
-                                     solves follow the same bits.  Default: all
-                                     three directions (7); setting ROWS sets it
-                                     to 0 */
+                                     solves follow the same bits.  Default: the
+                                     directions where it is the faster form, by the
+                                     lines' length and number, forward and transposed
+                                     apart (npbmz_describe's cols=); setting ROWS
+                                     sets it to 0 */
 int npbmz_set_schedule(npbmz_ctx* ctx, int32_t which, int32_t value);
 
 /* Describe the schedule currently in use (for logs); writes a NUL-terminated

@@ -280,6 +280,7 @@ struct npbmz_ctx {
   bool sp_twist_ok[3] = {false, false, false};  // SP: every line of direction d has >= 4 unknowns
   int solve_rows = 0;             // BT, FMA only: bit d set: solve_rows_kernel (wins over twist);
   int solve_cols = 0;             // BT, FMA only: bit d set: solve_cols_kernel (wins over rows)
+  int adj_cols = 0;               // the same for the transposed solves; set together
   int cus = 256;                  // the device's compute units
                                   // set at creation by size
   int halfmax[3] = {0, 0, 0};     // rows of the longer half of the longest line per direction
@@ -802,6 +803,48 @@ int k_add(npbmz_ctx* ctx, int zone) {
 // issued together).
 bool rows_long(const npbmz_ctx& c, int d) {
   return c.t_row[d].n > 4 * c.cus && c.halfmax[d] > kRowRLong;
+}
+
+// Where BT runs the columns solve by default: nearly everywhere (us for the
+// three solves of a step, rows / columns: class S 29.2 / 21.0, B 276 / 233, C
+// 1055 / 902; 122 / 104 on 131x97x23 in 3x2 zones), but not where most of long
+// lines' reduced rows are spilled and the spill no longer fits the 256 MB
+// last-level cache beside u and rhs: its spill costs more than that of the
+// rows kernel.  By the mean length L of a direction's lines, us along x / y / z, rows and
+// columns: 8 M points, L = 40 768 / 725 / 825 and 676 / 639 / 752, 56 833 /
+// 760 / 857 and 836 / 780 / 892, 64 833 / 769 / 848 and 866 / 811 / 899, 128 945 / 898 /
+// 952 and 1020 / 973 / 1083; 1 M points (up to 180 MB spilled), 64 117 / 116 /
+// 136 and 94 / 89 / 98, 128 137 / 131 / 139 and 120 / 105 / 114; 1.5 M, 64 (213
+// MB) 168 / 155 / 177 and 177 / 175 / 196.  Nor where the columns' waves are
+// just over one round of the chip (eight a CU, five lines each) and the rows'
+// within one (12 lines on two waves): 1.5 M points, 128 192 / 178 / 191 and 242
+// / 244 / 270, 1 M, 80 108 / 103 / 108 and 113 / 103 / 114.
+// The transposed columns solve gives way to the two-sided one (two waves a
+// task of 64 lines), along y and z, for long lines once that has tasks for five
+// eighths of the CUs: us along y / z, two-sided and columns, 1 M points, L =
+// 80 127 / 123 and 130 / 156, 104 (150 tasks) 158 / 144 and 122 / 137; 1.5 M,
+// 128 206 / 217 and 251 / 259, 160 (147 tasks) 244 / 225 and 216 / 219; 4 M, 40
+// 363 / 379 and 353 / 354, 160 458 / 417 and 542 / 544.
+void choose_cols(npbmz_ctx& c) {
+  c.solve_cols = c.adj_cols = 0;
+  for (int d = 0; d < 3; ++d) {
+    int64_t lines = 0, rows = 0, cols = 0, dozen = 0, wave = 0, spill = 0;
+    for (int z = 0; z < c.nz_; ++z) {
+      const int64_t n = lines_of(&c, z, d);
+      const int len = d == 0 ? c.nx[z] : d == 1 ? c.ny[z] : c.nz[z];
+      const int64_t t = (n + fast::bt::kColLines - 1) / fast::bt::kColLines;
+      lines += n;
+      rows += n * len;
+      cols += t;
+      dozen += (n + fast::bt::kRowLines - 1) / fast::bt::kRowLines;
+      wave += (n + kLineNT - 1) / kLineNT;
+      spill += t * cols_spill((len - 1) / 2) * fast::bt::kColRow * (int64_t)sizeof(double);
+    }
+    const bool short_lines = rows <= 56 * lines;
+    const bool one_round = cols <= 8 * c.cus || dozen > 4 * c.cus;
+    if (short_lines || (spill <= 200000000 && one_round)) c.solve_cols |= 1 << d;
+    if (d == 0 || short_lines || 8 * wave <= 5 * c.cus) c.adj_cols |= 1 << d;
+  }
 }
 
 // Waves of SP's staged solve that a CU's LDS holds, for lines of at most nl
@@ -1375,7 +1418,7 @@ int k_adj_solve(npbmz_ctx* ctx, const double* us, const double* x, const double*
   if (t.n <= 0) return NPBMZ_OK;
   int grid = t.n;
   if (c.solve_grid[DIR] > 0) grid = std::min(t.n, c.solve_grid[DIR]);
-  if ((c.solve_cols >> DIR) & 1) {
+  if ((c.adj_cols >> DIR) & 1) {
     const Table& tc = c.t_col[DIR];
     const int gc = c.solve_grid[DIR] > 0 ? std::min(tc.n, c.solve_grid[DIR]) : tc.n;
     hipLaunchKernelGGL((fast::bt::adj_solve_cols_kernel<DIR, kColR>), dim3(gc), dim3(64),
@@ -1748,11 +1791,11 @@ void describe(npbmz_ctx* c) {
     for (int d = 0; d < 3; ++d)
       ring[d] = strict(c) || !((c->solve_rows >> d) & 1) ? 0 : rows_long(*c, d) ? kRowRLong : kRowR;
     snprintf(b, sizeof b,
-             "zones=%d order=%s solve_grid=%d/%d/%d pair=%d twist=%d rows=%d ring=%d/%d/%d cols=%d fp=%s",
+             "zones=%d order=%s solve_grid=%d/%d/%d pair=%d twist=%d rows=%d ring=%d/%d/%d cols=%d/%d fp=%s",
              c->nz_, c->largest_first ? "largest-first" : "natural", c->solve_grid[0],
              c->solve_grid[1], c->solve_grid[2], c->solve_pair, strict(c) ? 0 : c->solve_twist,
              strict(c) ? 0 : c->solve_rows, ring[0], ring[1], ring[2],
-             strict(c) ? 0 : c->solve_cols, strict(c) ? "strict" : "fma");
+             strict(c) ? 0 : c->solve_cols, strict(c) ? 0 : c->adj_cols, strict(c) ? "strict" : "fma");
   }
   c->sched = b;
 }
@@ -1961,10 +2004,8 @@ int npbmz_create(const npbmz_problem* p, int32_t flags, npbmz_ctx** out) {
     // class S 0.057 / 0.039 / 0.037, W 0.083 / 0.056 / 0.054, A 0.172 /
     // 0.120 / 0.120, B 0.397 / 0.304 / 0.296, C 1.421 / 1.243 / 1.236
     c.solve_rows = 7;
-    // and over it the columns kernel, which is faster in every direction (us
-    // for the three solves of a step, rows / columns: class S 29.2 / 21.0, B
-    // 276 / 233, C 1055 / 902; 122 / 104 on 131x97x23 in 3x2 zones)
-    c.solve_cols = 7;
+    // and over it the columns kernel where that is the faster one
+    choose_cols(c);
   }
   if (c.bench == NPBMZ_SP) {
     // default: two-sided solves wherever the staged form is taken (ms/step
@@ -2553,12 +2594,12 @@ int npbmz_set_schedule(npbmz_ctx* ctx, int32_t which, int32_t value) {
       if (c.bench != NPBMZ_BT || value < 0 || value > 7)
         return fail(ctx, NPBMZ_EINVAL, "BT rows-over-lanes solve mask is 0..7");
       c.solve_rows = value;
-      c.solve_cols = 0;  // the rows kernel, or what it gives way to, as asked
+      c.solve_cols = c.adj_cols = 0;  // the rows kernel, or what it gives way to, as asked
       break;
     case NPBMZ_SCHED_SOLVE_COLS:
       if (c.bench != NPBMZ_BT || value < 0 || value > 7)
         return fail(ctx, NPBMZ_EINVAL, "BT columns solve mask is 0..7");
-      c.solve_cols = value;
+      c.solve_cols = c.adj_cols = value;
       break;
     case NPBMZ_SCHED_RHS_EXCH:
       if (c.bench == NPBMZ_LU || value < 0 || value > 1)

@@ -108,3 +108,57 @@ def test_columns_adjoint_tracks_the_two_sided_one(gpu, grid, zones, ratio):
         assert np.isfinite(a[k]).all()
         assert np.abs(a[k] - b[k]).max() <= 1e-12 * np.abs(a[k]).max(), k
         assert np.array_equal(b[k], c[k]), k
+
+
+# (grid, zones, ratio), the directions solved by columns (bit d) forward and
+# transposed: the classes and a grid between them; just over one round of
+# columns waves along x, within one of rows waves; long lines whose spill
+# leaves the last-level cache; the same along x only, short lines along y, and
+# many medium ones along z
+ROUTES = [
+    ("S", 7, 7), ("A", 7, 7), ("B", 7, 7), ("C", 7, 7),
+    (((131, 97, 23), (3, 2), 2.2), 7, 7),
+    (((80, 112, 112), (1, 1), 1.0), 6, 7),
+    (((200, 200, 200), (1, 1), 1.0), 0, 1),
+    (((400, 40, 64), (1, 1), 1.0), 6, 3),
+]
+
+
+@pytest.mark.parametrize("problem,forward,transposed", ROUTES)
+def test_columns_where_they_are_the_faster_ones(gpu, problem, forward, transposed):
+    if isinstance(problem, str):
+        z = gpu.zones_for("BT", problem)[0]
+    else:
+        grid, zones, ratio = problem
+        z = gpu.zone_setup(*zones, *grid, ratio)
+    ctx = gpu.Context("BT", z, 0.0003)
+    assert "cols=%d/%d" % (forward, transposed) in ctx.describe(), ctx.describe()
+    ctx.close()
+    ctx = gpu.Context("BT", z, 0.0003, strict=True)
+    assert "cols=0/0" in ctx.describe()
+    ctx.close()
+
+
+def test_directions_on_different_solves_agree(gpu):
+    """A default schedule with rows along x and columns along y and z, and
+    with columns and the two-sided solve transposed, against the two-sided
+    solve in all (the bounds of the tests above; a step small enough that
+    noise on 400 points along x decays)."""
+    N = gpu.native
+    for grid in ((80, 112, 112), (400, 40, 64)):
+        u, g = [], []
+        for default in (False, True):
+            ctx = gpu.Context("BT", gpu.zone_setup(1, 1, *grid, 1.0), 0.00003)
+            if not default:
+                ctx.set_schedule(N.SCHED_SOLVE_ROWS, 0)
+            ctx.init_exact()
+            u0 = ctx.get_all(0)
+            rng = np.random.default_rng(5)
+            ctx.put_all(0, u0 * (1.0 + 0.02 * rng.uniform(-1.0, 1.0, u0.size)))
+            g.append(ctx.adjoint(2, 1, np.random.default_rng(3).random(ctx.size)))
+            ctx.step(3, "graph")
+            u.append(ctx.get_all(0))
+            ctx.close()
+        assert np.abs(u[1] - u[0]).max() <= 1e-14 * np.abs(u[0]).max()
+        for k in ("grad_u0", "grad_forcing"):
+            assert np.abs(g[1][k] - g[0][k]).max() <= 1e-12 * np.abs(g[0][k]).max(), k
