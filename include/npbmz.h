@@ -190,7 +190,9 @@ int npbmz_tune(npbmz_ctx* ctx, int32_t budget_ms);
                                     where a workgroup's slots fit 448 threads;
                                     otherwise hyperplane launches).  Default
                                     with FMA arithmetic: 2 where a zone's padded
-                                    hyperplane has more than 256 slots, else 1;
+                                    hyperplane has more than 256 slots in rows of at
+                                    most 358 (ny up to 359), else 1 up to 32768
+                                    interior points;
                                     strict: 1 for zones of at most 32768
                                     interior points, else 0 */
 #define NPBMZ_SCHED_LU_THREADS 1 /* 128, 256 or 512 threads per zone workgroup

@@ -237,6 +237,7 @@ constexpr int kMaxSolveGrid = 65536; // largest persistent solve grid accepted
 enum { kSweepPlane = 0, kSweepZone = 1, kSweepTiles = 2 };
 constexpr int kMaxTiles = 8;    // tiles per zone of the pipelined sweep
 constexpr int kMaxGroups = 16;  // workgroups per zone its tiles may take
+constexpr int kTileRow = 358;   // slots of the longest row the tiles are the default for
 
 // A task table on the device plus, per zone, the range of its tasks; freed
 // with the context that holds it.
@@ -1225,23 +1226,28 @@ int k_lu_sweep_t(npbmz_ctx* ctx, int zone, bool* upd = nullptr) {
                          z0, nzl, nzp, g.G, g.rpt, g.parts, c.lu_kb, g.steps, c.txbuf, cn, dn, ef, c.lu_spin,
                          xc, c.lk);
     };
-    // the hand-off form: XCD-local with 4 or 8 doubles of a row per lane, or
-    // agent-scope
-    auto by_form = [&](auto k4, auto k8, auto agent) {
-      if (ho == 0) go(agent);
-      else if (g.SJ * 5 <= 4 * 64) go(k4);
-      else go(k8);
+    // the hand-off form: XCD-local or agent-scope, by a row's doubles per lane
+    auto by_form = [&](auto k4, auto k8, auto wide, auto agent8, auto agent_wide) {
+      const int per = (g.SJ * 5 + 63) / 64;
+      if (ho == 0) per <= 8 ? go(agent8) : go(agent_wide);
+      else if (per <= 4) go(k4);
+      else per <= 8 ? go(k8) : go(wide);
     };
     auto by_size = [&](auto nt) {
-      constexpr int NT = decltype(nt)::value;
-      if (UPPER && upd)
-        by_form(fast::lu::sweep_tile_kernel<UPPER, NT, true, 4, true>,
-                fast::lu::sweep_tile_kernel<UPPER, NT, true, 8, true>,
-                fast::lu::sweep_tile_kernel<UPPER, NT, false, 8, true>);
-      else
-        by_form(fast::lu::sweep_tile_kernel<UPPER, NT, true, 4>,
-                fast::lu::sweep_tile_kernel<UPPER, NT, true, 8>,
-                fast::lu::sweep_tile_kernel<UPPER, NT, false, 8>);
+      constexpr int NT = decltype(nt)::value, KW = NT == 128 ? 10 : 20;
+      if constexpr (UPPER) {
+        if (upd)
+          return by_form(fast::lu::sweep_tile_kernel<UPPER, NT, true, 4, true>,
+                         fast::lu::sweep_tile_kernel<UPPER, NT, true, 8, true>,
+                         fast::lu::sweep_tile_kernel<UPPER, NT, true, KW, true>,
+                         fast::lu::sweep_tile_kernel<UPPER, NT, false, 8, true>,
+                         fast::lu::sweep_tile_kernel<UPPER, NT, false, KW, true>);
+      }
+      by_form(fast::lu::sweep_tile_kernel<UPPER, NT, true, 4>,
+              fast::lu::sweep_tile_kernel<UPPER, NT, true, 8>,
+              fast::lu::sweep_tile_kernel<UPPER, NT, true, KW>,
+              fast::lu::sweep_tile_kernel<UPPER, NT, false, 8>,
+              fast::lu::sweep_tile_kernel<UPPER, NT, false, KW>);
     };
     if (g.nt == 128) by_size(std::integral_constant<int, 128>{});
     else if (g.nt == 256) by_size(std::integral_constant<int, 256>{});
@@ -1893,11 +1899,16 @@ int npbmz_create(const npbmz_problem* p, int32_t flags, npbmz_ctx** out) {
     if (interior > 32768) c.lu_sweep = kSweepPlane;
     else c.lu_nt = 512;
     // with FMA arithmetic, zones whose padded hyperplane exceeds 256 slots
-    // run as pipelined tiles of at most 256 slots each (below): both sweeps,
-    // us, one workgroup against tiles: class A (31x15 slots) 229 and 140;
-    // class B (51x16), whose hyperplane fits no workgroup, 1085 with
-    // hyperplane launches and 289.  Smaller ones gain little: 23x9 104 and 95,
-    // 19x11 83 and 86, class W (15x7) 47 and 60.
+    // run as pipelined tiles (below): both sweeps, us, one workgroup against
+    // tiles, 16 zones of 30 points along x: 13x13 slots 89 and 104, 23x9 103
+    // and 101, 23x10 108 and 112, 32x8 119 and 120, 16x16 116 and 111; over
+    // 256 slots the workgroup is of 512 threads: 20x14 172 and 113, 31x15 213
+    // and 135; class B (51x16), whose hyperplane fits no workgroup, 1085 with
+    // hyperplane launches and 289.  Up to kTileRow slots a row: of longer
+    // ones the hand-off loads in a second batch in each step, and ms per
+    // iteration with hyperplane launches and tiles, 4 zones of 60 points along
+    // x, 5 / 15 rows: 215 slots 2.06 / 2.22 and 0.80 / 1.06, 350 3.09 / 3.33
+    // and 1.93 / 2.59, 400 3.47 / 3.75 and 2.93 / 3.88
     // hyperplane forwarding: with FMA arithmetic the padded-halo sweep in
     // the smallest workgroup that holds a zone's padded hyperplane; strict
     // arithmetic has no padded-halo form: rsd and u through LDS from 128
@@ -1977,18 +1988,24 @@ int npbmz_create(const npbmz_problem* p, int32_t flags, npbmz_ctx** out) {
       // (the padded sweeps' smaller workgroups take under 64 KiB)
       grant(fast::lu::sweep_tile_kernel<false, 448, true, 4>);
       grant(fast::lu::sweep_tile_kernel<false, 448, true, 8>);
+      grant(fast::lu::sweep_tile_kernel<false, 448, true, 20>);
       grant(fast::lu::sweep_tile_kernel<false, 448, false, 8>);
+      grant(fast::lu::sweep_tile_kernel<false, 448, false, 20>);
       grant(fast::lu::sweep_tile_kernel<true, 448, true, 4>);
       grant(fast::lu::sweep_tile_kernel<true, 448, true, 8>);
+      grant(fast::lu::sweep_tile_kernel<true, 448, true, 20>);
       grant(fast::lu::sweep_tile_kernel<true, 448, false, 8>);
+      grant(fast::lu::sweep_tile_kernel<true, 448, false, 20>);
       grant(fast::lu::sweep_tile_kernel<true, 448, true, 4, true>);
       grant(fast::lu::sweep_tile_kernel<true, 448, true, 8, true>);
+      grant(fast::lu::sweep_tile_kernel<true, 448, true, 20, true>);
       grant(fast::lu::sweep_tile_kernel<true, 448, false, 8, true>);
+      grant(fast::lu::sweep_tile_kernel<true, 448, false, 20, true>);
       (void)hipGetLastError();
       if (ok) c.max_lds = (size_t)v;
     }
     const int slots = (c.ny[0] - 1) * (c.nz[0] - 1);
-    if (slots > 256 && !strict(ctx)) {
+    if (slots > 256 && c.ny[0] - 1 <= kTileRow && !strict(ctx)) {
       const int prev = c.lu_sweep;
       c.lu_sweep = kSweepTiles;
       c.lu_tiles = std::min(kMaxTiles, (slots + 255) / 256);
