@@ -1766,7 +1766,7 @@ void describe(npbmz_ctx* c) {
   if (c->bench == NPBMZ_LU && c->lu_sweep == kSweepTiles && lu_tiles_ok(c)) {
     const TileGeom g = tile_geom(c);
     snprintf(b, sizeof b, "zones=%d sweep=pipelined-tiles tiles=%d batch=%d nt=%d handoff=%s groups=%d exch=%s fp=%s",
-             c->nz_, g.W, c->lu_kb, g.nt * g.parts, tile_handoff(c) != 0 ? "xcd-local" : "agent", g.G,
+             c->nz_, g.W, c->lu_kb, g.nt, tile_handoff(c) != 0 ? "xcd-local" : "agent", g.G,
              (c->flags & NPBMZ_FLAG_LU_NPB_EXCH) ? "npb" : "reference",
              strict(c) ? "strict" : "fma");
   } else if (c->bench == NPBMZ_LU)

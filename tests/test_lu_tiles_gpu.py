@@ -219,14 +219,14 @@ def test_tile_knobs_are_validated(gpu):
 
 def test_default_sweeps_by_zone_size(gpu):
     """The library's defaults: zones whose padded hyperplane exceeds 256
-    slots run pipelined tiles of at most 256 slots (class A, 31x15 slots: 2
-    tiles; class B, 51x16: 4), smaller ones one workgroup per zone (class
-    W); strict arithmetic (no tile kernel) keeps the padded-halo-free zone
+    slots run pipelined tiles (class A, 31x15 slots: 2 tiles; class B, 51x16:
+    4), each as workgroups of at most 128 slots, nt, and the hand-off wave (4
+    and 8 a zone); smaller ones run one workgroup per zone (class W); strict arithmetic (no tile kernel) keeps the padded-halo-free zone
     workgroups at class A and hyperplane launches at class B."""
     for cls, strict, want in (("W", False, "zone-workgroup"),
-                              ("A", False, "pipelined-tiles tiles=2 batch=4 nt=256 handoff=xcd-local"),
+                              ("A", False, "pipelined-tiles tiles=2 batch=4 nt=128 handoff=xcd-local groups=4"),
                               ("A", True, "zone-workgroup"),
-                              ("B", False, "pipelined-tiles tiles=4 batch=4 nt=256 handoff=xcd-local"),
+                              ("B", False, "pipelined-tiles tiles=4 batch=4 nt=128 handoff=xcd-local groups=8"),
                               ("B", True, "hyperplane-launch")):
         zones, p = gpu.zones_for("LU", cls)
         ctx = gpu.Context("LU", zones, p.dt, omega=1.2, npb_exchange=True, strict=strict)
