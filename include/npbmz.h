@@ -170,14 +170,16 @@ int npbmz_zone_norms(npbmz_ctx* ctx, double* rms_rhs, double* rms_err);
  * schedules for about budget_ms in total, one knob after another (each knob
  * keeps its fastest value while the next is tried): for BT/SP the task order
  * (largest zones first, and in each solve direction the zones with the
- * longest lines first; or natural order), the line-solve kernel per
- * direction (BT: one wave per 64 lines, a builder/eliminator wave pair, or,
- * with FMA arithmetic, the two-sided elimination)
- * and the solve grid (one block per 64 lines, or a persistent grid of 1024
- * blocks striding over them); for LU the SSOR sweep schedule (one workgroup
- * of 128/256/512 threads per zone walking all hyperplanes, or one launch per
- * i+j+k hyperplane over all zones).  The state is restored afterwards; the
- * chosen schedule is kept in the context for all modes.  No counterpart in
+ * longest lines first; or natural order), the forward line-solve kernel per
+ * direction (with FMA arithmetic BT's columns, rows and two-sided solves and
+ * SP's two-sided ones; BT's one wave per 64 lines or builder/eliminator wave
+ * pair; not those that the chosen ones override) and the solve grid (one block
+ * per task, or a persistent grid of 1024 blocks striding over them); for LU
+ * the SSOR sweep schedule (one workgroup of 128/256/512 threads per zone
+ * walking all hyperplanes, pipelined tiles, or one launch per i+j+k hyperplane
+ * over all zones).  The steps timed are forward ones: the adjoint's
+ * transposed solves keep their kernels.  The state is restored afterwards;
+ * the chosen schedule is kept in the context for all modes.  No counterpart in
  * the reference (its zone->thread schedule is Threads.@threads over zones,
  * src/BT/bt-node.jl:318). */
 int npbmz_tune(npbmz_ctx* ctx, int32_t budget_ms);

@@ -2457,15 +2457,32 @@ int npbmz_tune(npbmz_ctx* ctx, int32_t budget_ms) {
              {NPBMZ_SCHED_LU_TILE_BATCH, {1, 2, 4}}};
   } else {
     knobs.push_back({-1, {1, 0}});
-    if (c.bench == NPBMZ_BT) knobs.push_back({NPBMZ_SCHED_SOLVE_PAIR, {0, 2, 3, 7}});
-    if (!strict(ctx)) knobs.push_back({NPBMZ_SCHED_SOLVE_TWIST, {0, 1, 3, 7}});
-    if (c.bench == NPBMZ_BT && !strict(ctx))
-      knobs.push_back({NPBMZ_SCHED_SOLVE_ROWS, {0, 1, 3, 7}});
-    if (c.bench == NPBMZ_BT && !strict(ctx))  // after ROWS, which sets it to 0
+    // BT's solves from the one that overrides the others down
+    if (c.bench == NPBMZ_BT && !strict(ctx)) {
       knobs.push_back({NPBMZ_SCHED_SOLVE_COLS, {0, 1, 3, 7}});
+      knobs.push_back({NPBMZ_SCHED_SOLVE_ROWS, {0, 1, 3, 7}});
+    }
+    if (!strict(ctx)) knobs.push_back({NPBMZ_SCHED_SOLVE_TWIST, {0, 1, 3, 7}});
+    if (c.bench == NPBMZ_BT) knobs.push_back({NPBMZ_SCHED_SOLVE_PAIR, {0, 2, 3, 7}});
     knobs.push_back({NPBMZ_SCHED_SOLVE_GRID, {0, 1024}});
     knobs.push_back({NPBMZ_SCHED_RHS_EXCH, {1, 0}});
   }
+  // knobs that do nothing under what is chosen so far keep their values:
+  // trials of one schedule against itself would pick by noise
+  auto idle = [&](int which) {
+    const int over = strict(ctx) ? 0 : c.solve_cols;
+    switch (which) {
+      case NPBMZ_SCHED_LU_THREADS:
+      case NPBMZ_SCHED_LU_FORWARD: return c.lu_sweep != kSweepZone;
+      case NPBMZ_SCHED_LU_TILES:
+      case NPBMZ_SCHED_LU_TILE_BATCH: return c.lu_sweep != kSweepTiles || !lu_tiles_ok(&c);
+      case NPBMZ_SCHED_SOLVE_ROWS: return over == 7;
+      case NPBMZ_SCHED_SOLVE_TWIST: return c.bench == NPBMZ_BT && (over | c.solve_rows) == 7;
+      case NPBMZ_SCHED_SOLVE_PAIR:
+        return !strict(ctx) && (over | c.solve_rows | c.solve_twist) == 7;
+      default: return false;
+    }
+  };
   auto get = [&](int which) -> int {
     switch (which) {
       case NPBMZ_SCHED_LU_SWEEP: return c.lu_sweep;
@@ -2484,13 +2501,14 @@ int npbmz_tune(npbmz_ctx* ctx, int32_t budget_ms) {
   };
   auto set = [&](int which, int v) -> int {
     if (which >= 0) {
-      if ((which == NPBMZ_SCHED_LU_THREADS || which == NPBMZ_SCHED_LU_FORWARD) &&
-          c.lu_sweep != kSweepZone)
-        return NPBMZ_OK;
-      if ((which == NPBMZ_SCHED_LU_TILES || which == NPBMZ_SCHED_LU_TILE_BATCH) &&
-          c.lu_sweep != kSweepTiles)
-        return NPBMZ_OK;
-      return npbmz_set_schedule(ctx, which, v);
+      // the steps timed are forward ones: the transposed solves keep theirs,
+      // and ROWS leaves COLS alone
+      const int cols = c.solve_cols, adj_cols = c.adj_cols, adj_twist = c.adj_twist;
+      const int r = npbmz_set_schedule(ctx, which, v);
+      if (which == NPBMZ_SCHED_SOLVE_ROWS) c.solve_cols = cols;
+      c.adj_cols = adj_cols;
+      c.adj_twist = adj_twist;
+      return r;
     }
     c.largest_first = v == 1;
     if (c.largest_first) c.order = cost_order(c);
@@ -2507,7 +2525,7 @@ int npbmz_tune(npbmz_ctx* ctx, int32_t budget_ms) {
       hipMemcpyAsync(sr, c.rhs, fb, hipMemcpyDeviceToDevice, c.stream) != hipSuccess)
     rc = fail(ctx, NPBMZ_EHIP, "tune save");
   size_t trials = 0;
-  for (auto& k : knobs) trials += k.values.size();
+  for (auto& k : knobs) trials += idle(k.which) ? 0 : k.values.size();
   const double per = std::max(1.0, double(budget_ms) / trials);
   auto trial = [&](double& t) -> int {
     double ms = 0.0, tot = 0.0;
@@ -2526,7 +2544,10 @@ int npbmz_tune(npbmz_ctx* ctx, int32_t budget_ms) {
   };
   for (auto& k : knobs) {
     if (rc) break;
+    if (idle(k.which)) continue;
     int best_v = get(k.which);
+    if (std::find(k.values.begin(), k.values.end(), best_v) == k.values.end())
+      k.values.push_back(best_v);
     double best = 1e300;
     for (int v : k.values) {
       double t = 0.0;

@@ -79,6 +79,28 @@ def test_tune_keeps_the_fields_and_the_tuned_run_verifies(gpu, bench):
     ctx.close()
 
 
+def test_tune_leaves_knobs_that_do_nothing_and_the_transposed_solves(gpu):
+    """With BT's columns or rows solves in every direction the two-sided and
+    the wave-pair solves never run: the tuner leaves their masks (values it
+    does not try itself) as they were.  Its trials are forward steps, so the
+    transposed solves keep theirs."""
+    N = gpu.native
+    zones, p = gpu.zones_for("BT", "W")
+    ctx = gpu.Context("BT", zones, p.dt)
+    ctx.set_schedule(N.SCHED_SOLVE_TWIST, 5)
+    ctx.set_schedule(N.SCHED_SOLVE_PAIR, 1)
+    ctx.set_schedule(N.SCHED_SOLVE_COLS, 6)
+    ctx.init_exact()
+    ctx.tune(200)
+    sched = ctx.describe()
+    ctx.close()
+    now = dict(x.split("=") for x in sched.split())
+    cols, transposed = now["cols"].split("/")
+    assert transposed == "6", sched
+    if int(cols) | int(now["rows"]) == 7:
+        assert now["twist"] == "5" and now["pair"] == "1", sched
+
+
 @pytest.mark.parametrize("bench", ["BT", "SP"])
 def test_schedule_change_discards_both_step_graphs(gpu, bench):
     """Graph mode replays a captured eight-step graph and a one-step graph;
