@@ -498,10 +498,6 @@ int lines_of(const npbmz_ctx* c, int z, int dir) {
                   : dir == 1 ? (c->nx[z] - 2) * (c->nz[z] - 2) : (c->nx[z] - 2) * (c->ny[z] - 2);
 }
 
-// Build a task table: zones in `order`, each zone's `count(z)` items cut into
-// tasks of `per` items.  The new device table is allocated before the old
-// one is freed, and t changes only on success, so a failure leaves the
-// previous table in place and usable.
 // solve_cols_kernel's reduced rows for half lines of at most halfmax rows:
 // the last kColR of a half in registers (none of a half shorter than that),
 // up to kColLds in LDS, the rest spilled.
@@ -528,6 +524,10 @@ fast::bt::ColK make_col_constants(const StencilK& K, int d) {
   return k;
 }
 
+// Build a task table: zones in `order`, each zone's `count(z)` items cut into
+// tasks of `per` items.  The new device table is allocated before the old
+// one is freed, and t changes only on success, so a failure leaves the
+// previous table in place and usable.
 template <class F>
 int build_table(npbmz_ctx* ctx, Table& t, const std::vector<int>& order, int per, F count) {
   std::vector<Task> h;
@@ -807,25 +807,26 @@ bool rows_long(const npbmz_ctx& c, int d) {
 }
 
 // Where BT runs the columns solve by default: nearly everywhere (us for the
-// three solves of a step, rows / columns: class S 29.2 / 21.0, B 276 / 233, C
-// 1055 / 902; 122 / 104 on 131x97x23 in 3x2 zones), but not where most of long
-// lines' reduced rows are spilled and the spill no longer fits the 256 MB
-// last-level cache beside u and rhs: its spill costs more than that of the
-// rows kernel.  By the mean length L of a direction's lines, us along x / y / z, rows and
-// columns: 8 M points, L = 40 768 / 725 / 825 and 676 / 639 / 752, 56 833 /
-// 760 / 857 and 836 / 780 / 892, 64 833 / 769 / 848 and 866 / 811 / 899, 128 945 / 898 /
-// 952 and 1020 / 973 / 1083; 1 M points (up to 180 MB spilled), 64 117 / 116 /
-// 136 and 94 / 89 / 98, 128 137 / 131 / 139 and 120 / 105 / 114; 1.5 M, 64 (213
-// MB) 168 / 155 / 177 and 177 / 175 / 196.  Nor where the columns' waves are
-// just over one round of the chip (eight a CU, five lines each) and the rows'
-// within one (12 lines on two waves): 1.5 M points, 128 192 / 178 / 191 and 242
-// / 244 / 270, 1 M, 80 108 / 103 / 108 and 113 / 103 / 114.
+// three solves of a step, rows and columns: class S 36 and 28, B 245 and 211,
+// C 995 and 866; 120 and 101 on 131x97x23 in 3x2 zones), but not where most
+// of long lines' reduced rows are spilled and the spill no longer fits the
+// 256 MB last-level cache beside u and rhs: there its spill costs more than
+// the rows kernel's. By the mean length L of a direction's lines, us along x
+// / y / z, rows and columns: 8 M points, L = 40 768 / 725 / 825 and 676 / 639
+// / 752, 56 833 / 760 / 857 and 836 / 780 / 892, 64 833 / 769 / 848 and 866 /
+// 811 / 899, 128 945 / 898 / 952 and 1020 / 973 / 1083; 1 M points (up to 180
+// MB spilled), 64 117 / 116 / 136 and 94 / 89 / 98, 128 137 / 131 / 139 and
+// 120 / 105 / 114; 1.5 M, 64 (213 MB) 168 / 155 / 177 and 177 / 175 / 196.
+// Nor where the columns' waves are just over one round of the chip (eight a
+// CU, five lines each) and the rows' within one (12 lines on two waves): 1.5
+// M points, 128 192 / 178 / 191 and 242 / 244 / 270; 1 M, 80 108 / 103 / 108
+// and 113 / 103 / 114.
 // The transposed columns solve gives way to the two-sided one (two waves a
-// task of 64 lines), along y and z, for long lines once that has tasks for five
-// eighths of the CUs: us along y / z, two-sided and columns, 1 M points, L =
-// 80 127 / 123 and 130 / 156, 104 (150 tasks) 158 / 144 and 122 / 137; 1.5 M,
-// 128 206 / 217 and 251 / 259, 160 (147 tasks) 244 / 225 and 216 / 219; 4 M, 40
-// 363 / 379 and 353 / 354, 160 458 / 417 and 542 / 544.
+// task of 64 lines), along y and z, for long lines once that has tasks for
+// five eighths of the CUs: us along y / z, two-sided and columns, 1 M points,
+// L = 80 127 / 123 and 130 / 156, 104 (150 tasks) 158 / 144 and 122 / 137;
+// 1.5 M, 128 206 / 217 and 251 / 259, 160 (147 tasks) 244 / 225 and 216 /
+// 219; 4 M, 40 363 / 379 and 353 / 354, 160 458 / 417 and 542 / 544.
 void choose_cols(npbmz_ctx& c) {
   c.solve_cols = c.adj_cols = 0;
   for (int d = 0; d < 3; ++d) {

@@ -71,9 +71,11 @@ def test_handoff_forms_and_modes_agree_bitwise(gpu, dims):
     replays, and both exchanges' planes per form: the same values move."""
     knobs = dict(TILES, LU_TILES=4)
     for npb in (False, True):
-        ref, _ = _run(gpu, dims, knobs, npb=npb)
+        ref, desc = _run(gpu, dims, knobs, npb=npb)
+        assert "handoff=xcd-local" in desc, desc
         for kw in (dict(knobs, LU_HANDOFF=0), dict(knobs, LU_TILE_BATCH=1), dict(knobs, LU_TILES=8)):
-            got, _ = _run(gpu, dims, kw, mode="graph" if "LU_TILE_BATCH" in kw else "perzone", npb=npb)
+            got, desc = _run(gpu, dims, kw, mode="graph" if "LU_TILE_BATCH" in kw else "perzone", npb=npb)
+            assert ("handoff=agent" if "LU_HANDOFF" in kw else "handoff=xcd-local") in desc, desc
             assert np.array_equal(got[0], ref[0]) and np.array_equal(got[1], ref[1]), (kw, npb)
 
 
