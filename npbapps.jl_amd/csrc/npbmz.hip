@@ -865,7 +865,7 @@ int64_t staged_waves(int nl, int lds) {
 //    lines of L points in r rounds of w waves per CU.  The two-wave solve,
 //    taken where it has fewer tasks than CUs, takes 0.6 to 0.7 L whatever
 //    their number, so the line is at 2 (w + 1) tasks per CU.  us along y, two
-//    waves and staged: 1 M points, L = 128 81 and 73, 160 98 and 100; 1.5 M, 96
+//    waves and staged: 1 M points, L = 128 81 and 73, 156 96 and 100; 1.5 M, 96
 //    69 and 83, 128 83 and 97, 200 123 and 155; 2 M, 140 95 and 132, 300
 //    180 and 183;
 //  - against the one-wave solve, taken from there on, it loses with one wave
