@@ -818,9 +818,11 @@ bool rows_long(const npbmz_ctx& c, int d) {
 // MB spilled), 64 117 / 116 / 136 and 94 / 89 / 98, 128 137 / 131 / 139 and
 // 120 / 105 / 114; 1.5 M, 64 (213 MB) 168 / 155 / 177 and 177 / 175 / 196.
 // Nor where the columns' waves are just over one round of the chip (eight a
-// CU, five lines each) and the rows' within one (12 lines on two waves): 1.5
-// M points, 128 192 / 178 / 191 and 242 / 244 / 270; 1 M, 80 108 / 103 / 108
-// and 113 / 103 / 114.
+// CU, five lines each) and the rows' within one (12 lines on two waves), with
+// lines of one length: 1.5 M points, 128 192 / 178 / 191 and 242 / 244 / 270;
+// 1 M, 80 108 / 103 / 108 and 113 / 103 / 114. Of uneven lines the last
+// round's are the shortest: 154x233x27 in 2x8 zones, 28 to 126 points along
+// x, 117 and 98.
 // The transposed columns solve gives way to the two-sided one (two waves a
 // task of 64 lines), along y and z, for long lines once that has tasks for
 // five eighths of the CUs: us along y / z, two-sided and columns, 1 M points,
@@ -831,10 +833,13 @@ void choose_cols(npbmz_ctx& c) {
   c.solve_cols = c.adj_cols = 0;
   for (int d = 0; d < 3; ++d) {
     int64_t lines = 0, rows = 0, cols = 0, dozen = 0, wave = 0, spill = 0;
+    int64_t shortest = INT64_MAX, longest = 0;
     for (int z = 0; z < c.nz_; ++z) {
       const int64_t n = lines_of(&c, z, d);
       const int len = d == 0 ? c.nx[z] : d == 1 ? c.ny[z] : c.nz[z];
       const int64_t t = (n + fast::bt::kColLines - 1) / fast::bt::kColLines;
+      shortest = std::min<int64_t>(shortest, len);
+      longest = std::max<int64_t>(longest, len);
       lines += n;
       rows += n * len;
       cols += t;
@@ -843,8 +848,9 @@ void choose_cols(npbmz_ctx& c) {
       spill += t * cols_spill((len - 1) / 2) * fast::bt::kColRow * (int64_t)sizeof(double);
     }
     const bool short_lines = rows <= 56 * lines;
-    const bool one_round = cols <= 8 * c.cus || dozen > 4 * c.cus;
-    if (short_lines || (spill <= 200000000 && one_round)) c.solve_cols |= 1 << d;
+    const bool just_over_a_round =
+        cols > 8 * c.cus && dozen <= 4 * c.cus && 8 * longest <= 9 * shortest;
+    if (short_lines || (spill <= 200000000 && !just_over_a_round)) c.solve_cols |= 1 << d;
     if (d == 0 || short_lines || 8 * wave <= 5 * c.cus) c.adj_cols |= 1 << d;
   }
 }

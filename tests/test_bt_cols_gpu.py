@@ -112,13 +112,15 @@ def test_columns_adjoint_tracks_the_two_sided_one(gpu, grid, zones, ratio):
 
 # (grid, zones, ratio), the directions solved by columns (bit d) forward and
 # transposed: the classes and a grid between them; just over one round of
-# columns waves along x, within one of rows waves; long lines whose spill
+# columns waves along x, within one of rows waves, with lines of one length
+# and uneven ones; long lines whose spill
 # leaves the last-level cache; the same along x only, short lines along y, and
 # many medium ones along z
 ROUTES = [
     ("S", 7, 7), ("A", 7, 7), ("B", 7, 7), ("C", 7, 7),
     (((131, 97, 23), (3, 2), 2.2), 7, 7),
     (((80, 112, 112), (1, 1), 1.0), 6, 7),
+    (((154, 233, 27), (2, 8), 4.43), 7, 7),
     (((200, 200, 200), (1, 1), 1.0), 0, 1),
     (((400, 40, 64), (1, 1), 1.0), 6, 3),
 ]
